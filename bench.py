@@ -8,7 +8,7 @@ A step is one brickwork layer: u3 on every qubit (3 SingleOps each), rzz on
 alternating nearest-neighbour pairs, one controlled x -- 105 or 106
 reference SingleOps.  --steps K layers of the depth-40 circuit are timed
 after --warmup W layers.  `value` counts reference SingleOps (u3 = 3), the
-unit the plain form launches one kernel for.
+unit the plain form rounds by.
 
 The roofline object reports the kernel class that dominates device time,
 from HIP events recorded on the register's stream around every launch in
@@ -52,6 +52,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 MFMA_PEAK_TFLOPS = {"f64": 78.6, "f32": 157.3}   # MI355X dense matrix-core peaks
+PLAIN_KERNELS = {"diag": "k_diag", "pair": "k_pair", "quad": "k_quad", "fused": "k_run"}   # of the plain form, by class
 METRIC = "gates/s + % HBM roofline at 30q FP64; served circuits/s at p50/p99 latency"
 
 
@@ -310,10 +311,10 @@ def tfim_leg(n, prec, plain_steps, fused_steps, per_step=False, dense=0, per_ste
                             "seconds": round(wall, 3), "norm_minus_1": norm - 1.0,
                             "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                                          "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
-                                         "kernel": "k_" + dom, "launches": d["launches"],
+                                         "kernel": PLAIN_KERNELS.get(dom, dom), "launches": d["launches"],
                                          "avg_ms": round(d["ms"] / d["launches"], 3)}}
-            log("tfim plain: %d SingleOps in %.2f s -> %.2f gates/s, k_%s %.0f GB/s; |psi|^2-1 = %.1e"
-                % (gates, wall, gates / wall, dom, ach, norm - 1.0))
+            log("tfim plain: %d SingleOps in %.2f s -> %.2f gates/s, %s %.0f GB/s; |psi|^2-1 = %.1e"
+                % (gates, wall, gates / wall, PLAIN_KERNELS.get(dom, dom), ach, norm - 1.0))
         out["fused"] = {}
         forms = [("whole", fused_steps, fused_steps)]
         if per_step or per_step_steps:
@@ -508,7 +509,7 @@ def serve_leg(requests, n_hi, slots, arena_gib, dense, plain=True, loads=(0.5, 0
 def batch_leg(registers, n_hi, prec, tile_cap, dense, steps, warmup, check, plain=True):
     """Batched uneven registers (n uniform in [10, n_hi], 20-400 mixed gates,
     seeded), each from |0>.  The plain form applies every register's circuit
-    one kernel per SingleOp, register after register; the batched form
+    SingleOp by SingleOp, register after register; the batched form
     compiles all circuits (tile_cap 0: autotuned tile caps and dense-phase
     thresholds) and runs them round by round as one hipGraph, `steps` runs
     timed.  value = SingleOps/s of the batched form over all registers."""
@@ -865,7 +866,7 @@ def main():
     per_launch_bytes = d["bytes"] / d["launches"]
     avg_ms = d["ms"] / d["launches"]
     achieved = per_launch_bytes / (avg_ms * 1e-3) / 1e9
-    kernel_name = {"diag": "k_diag", "pair": "k_pair", "quad": "k_quad"}.get(dom, dom)
+    kernel_name = PLAIN_KERNELS.get(dom, dom)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": load_traffic(kernel_name),
                 "traffic_source": "profiles/pmc_traffic.json (not measured in this run): rocprofv3 --pmc FETCH_SIZE "
@@ -912,7 +913,7 @@ def main():
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64",
         "data": "synthetic (seeded brickwork circuit, angles U[0,2pi))",
         "config": {"workload": label, "qubits": n, "state_gib": (16 << n) / 2**30, "singleops_timed": timed_gates,
-                   "form": "plain (one in-place kernel per SingleOp)", "step": "one brickwork layer (105-106 SingleOps)"},
+                   "form": "plain (SingleOps in queue order, each with its own rounding; runs of them share a pass)", "step": "one brickwork layer (105-106 SingleOps)"},
         "roofline": roofline,
         "all_kernels_gbs": round(all_bytes / all_ms / 1e6, 1) if all_ms else None,
         "fused": fused,

@@ -184,9 +184,11 @@ uint32_t qvnt_reg_num(const qvnt_reg* reg);                       /* QReg::num *
 uint64_t qvnt_reg_len(const qvnt_reg* reg);
 qvnt_prec qvnt_reg_prec(const qvnt_reg* reg);
 
-/* QReg::apply(&MultiOp) (quant.rs:376-395): the plain form — one in-place
- * kernel per SingleOp, in queue order, on the register's stream.  Results
- * equal the reference's out-of-place gather (dispatch.rs:32-47). */
+/* QReg::apply(&MultiOp) (quant.rs:376-395): the plain form -- every SingleOp
+ * in queue order with its own rounding, in place, on the register's stream.
+ * Results equal the reference's out-of-place gather (dispatch.rs:32-47).
+ * Consecutive SingleOps that mix few enough qubits share one pass over the
+ * state (timed as QVNT_K_FUSED); a single one runs as its own kernel. */
 int qvnt_reg_apply(qvnt_reg* reg, const qvnt_op* op);
 /* Same for a raw gate array (borrowed for the call). */
 int qvnt_reg_apply_gates(qvnt_reg* reg, const qvnt_gate* gates, size_t count);

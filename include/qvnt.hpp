@@ -229,7 +229,7 @@ public:
 
     uint32_t num() const { return q_num_; }
     uint64_t len() const { return qvnt_reg_len(h_); }
-    // QReg::apply: one kernel per SingleOp
+    // QReg::apply: every SingleOp in queue order, with its own rounding
     QReg& apply(const MultiOp& o) {
         check(qvnt_reg_apply(h_, o.handle()));
         return *this;

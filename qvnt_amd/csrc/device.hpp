@@ -15,6 +15,10 @@
 
 namespace qvnt {
 
+// The formulas run on the device; a CPU model of the kernels calls the same
+// code on the host.
+#define QVNT_HD __host__ __device__ __forceinline__
+
 template <class R>
 struct alignas(2 * sizeof(R)) cplx {
     R re, im;
@@ -23,23 +27,23 @@ using c64 = cplx<double>;
 using c32 = cplx<float>;
 
 template <class R>
-__device__ __forceinline__ cplx<R> cmul(cplx<R> a, cplx<R> b) {
+QVNT_HD cplx<R> cmul(cplx<R> a, cplx<R> b) {
     return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
 }
 template <class R>
-__device__ __forceinline__ cplx<R> cadd(cplx<R> a, cplx<R> b) { return {a.re + b.re, a.im + b.im}; }
+QVNT_HD cplx<R> cadd(cplx<R> a, cplx<R> b) { return {a.re + b.re, a.im + b.im}; }
 template <class R>
-__device__ __forceinline__ cplx<R> cneg(cplx<R> a) { return {-a.re, -a.im}; }
+QVNT_HD cplx<R> cneg(cplx<R> a) { return {-a.re, -a.im}; }
 template <class R>
-__device__ __forceinline__ cplx<R> cscale(cplx<R> a, R t) { return {a.re * t, a.im * t}; }
+QVNT_HD cplx<R> cscale(cplx<R> a, R t) { return {a.re * t, a.im * t}; }
 // math::rotate (src/math/mod.rs:41-50): i^q * z, q mod 4.
 template <class R>
-__device__ __forceinline__ cplx<R> rotate(cplx<R> z, uint64_t q) {
+QVNT_HD cplx<R> rotate(cplx<R> z, uint64_t q) {
     if (q & 2u) z = cneg(z);
     if (q & 1u) z = cplx<R>{-z.im, z.re};
     return z;
 }
-__device__ __forceinline__ unsigned dpopc(uint64_t x) { return (unsigned)__popcll(x); }
+QVNT_HD unsigned dpopc(uint64_t x) { return (unsigned)__builtin_popcountll(x); }
 
 // Bit positions inserted into a compact thread index to enumerate one
 // representative per orbit: `pos` ascending, then `set` ORed in (control
@@ -100,14 +104,14 @@ constexpr double kFrac1Sqrt2 = 0.70710678118654752440;
 // register's precision R (for R = double both conversions are the identity,
 // so FP64 registers round exactly like the reference).
 template <class R>
-__device__ __forceinline__ c64 up(cplx<R> p) { return c64{(double)p.re, (double)p.im}; }
+QVNT_HD c64 up(cplx<R> p) { return c64{(double)p.re, (double)p.im}; }
 template <class R>
-__device__ __forceinline__ cplx<R> down(c64 p) { return cplx<R>{(R)p.re, (R)p.im}; }
+QVNT_HD cplx<R> down(c64 p) { return cplx<R>{(R)p.re, (R)p.im}; }
 
 // ------------------------------------------------------------- diagonals
 // out[idx] = f(psi[idx]); kinds Z, S, T, RZ, RZZ, PHI.
 template <int K>
-__device__ __forceinline__ c64 f_diag64(const Par& g, uint64_t idx, c64 p) {
+QVNT_HD c64 f_diag64(const Par& g, uint64_t idx, c64 p) {
     if constexpr (K == QVNT_Z) {                                   // z.rs:15-21
         return (dpopc(idx & g.a) & 1u) ? cneg(p) : p;
     } else if constexpr (K == QVNT_S) {                            // s.rs:19-25
@@ -134,7 +138,7 @@ __device__ __forceinline__ c64 f_diag64(const Par& g, uint64_t idx, c64 p) {
     }
 }
 template <int K, class R>
-__device__ __forceinline__ cplx<R> f_diag(const Par& g, uint64_t idx, cplx<R> p) {
+QVNT_HD cplx<R> f_diag(const Par& g, uint64_t idx, cplx<R> p) {
     return down<R>(f_diag64<K>(g, idx, up(p)));
 }
 
@@ -142,7 +146,7 @@ __device__ __forceinline__ cplx<R> f_diag(const Par& g, uint64_t idx, cplx<R> p)
 // out[idx] = f(psi[idx], psi[idx ^ m]); `self` = psi[idx],
 // `other` = psi[idx ^ m] with m the orbit mask.
 template <int K>
-__device__ __forceinline__ c64 f_pair64(const Par& g, uint64_t idx, c64 self, c64 other) {
+QVNT_HD c64 f_pair64(const Par& g, uint64_t idx, c64 self, c64 other) {
     if constexpr (K == QVNT_X) {                                   // x.rs:15-17
         return other;
     } else if constexpr (K == QVNT_Y) {                            // y.rs:17-23
@@ -184,7 +188,7 @@ __device__ __forceinline__ c64 f_pair64(const Par& g, uint64_t idx, c64 self, c6
     }
 }
 template <int K, class R>
-__device__ __forceinline__ cplx<R> f_pair(const Par& g, uint64_t idx, cplx<R> self, cplx<R> other) {
+QVNT_HD cplx<R> f_pair(const Par& g, uint64_t idx, cplx<R> self, cplx<R> other) {
     return down<R>(f_pair64<K>(g, idx, up(self), up(other)));
 }
 
@@ -192,14 +196,14 @@ __device__ __forceinline__ cplx<R> f_pair(const Par& g, uint64_t idx, cplx<R> se
 // v[k] = psi[base | sel_k] with sel bits (b, a) = k; output for v-slot `s`.
 // h2.rs:22-38 for slot s, from the quad as seen from s: t0 = v[s],
 // t1 = v[s ^ 1], t2 = v[s ^ 2], t3 = v[s ^ 3].
-__device__ __forceinline__ c64 f_h2_rel(int s, c64 t0, c64 t1, c64 t2, c64 t3) {
+QVNT_HD c64 f_h2_rel(int s, c64 t0, c64 t1, c64 t2, c64 t3) {
     if (s & 1) { t0 = cneg(t0); t2 = cneg(t2); }
     if (s & 2) { t0 = cneg(t0); t1 = cneg(t1); }
     return cscale(cadd(cadd(cadd(t0, t1), t2), t3), 0.5);
 }
 
 template <int K>
-__device__ __forceinline__ c64 f_quad64(const Par& g, int s, const c64* v) {
+QVNT_HD c64 f_quad64(const Par& g, int s, const c64* v) {
     if constexpr (K == QVNT_H2) {                                  // h2.rs:22-38
         return f_h2_rel(s, v[s], v[s ^ 1], v[s ^ 2], v[s ^ 3]);
     } else {                                                       // u2.rs:22-49
@@ -212,7 +216,7 @@ __device__ __forceinline__ c64 f_quad64(const Par& g, int s, const c64* v) {
     }
 }
 template <int K, class R>
-__device__ __forceinline__ cplx<R> f_quad(const Par& g, int s, const cplx<R>* v) {
+QVNT_HD cplx<R> f_quad(const Par& g, int s, const cplx<R>* v) {
     const c64 w[4] = {up(v[0]), up(v[1]), up(v[2]), up(v[3])};
     return down<R>(f_quad64<K>(g, s, w));
 }

@@ -1,4 +1,5 @@
-// The plain form of QReg::apply: one in-place kernel per SingleOp.
+// The plain form of QReg::apply, one SingleOp: an in-place kernel per gate
+// kind (runs.hip applies several SingleOps in one pass, with these formulas).
 //
 // The reference gathers every output element from a read-only input buffer
 // (src/operator/atomic/dispatch.rs:32-47, multi/mod.rs:96-104), which needs

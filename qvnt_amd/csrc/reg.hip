@@ -287,11 +287,7 @@ int qvnt_reg_apply_gates(qvnt_reg* r, const qvnt_gate* gates, size_t count) {
         bool noop = false;
         if (int rc = check_gate(r->len, gates[i], &noop)) return rc;
     }
-    for (size_t i = 0; i < count; ++i) {
-        int rc = launch_gate(r, gates[i]);
-        if (rc) return rc;
-    }
-    return QVNT_OK;
+    return apply_plain(r, gates, count);
 }
 
 int qvnt_reg_apply_fused(qvnt_reg* r, const qvnt_op* op, uint32_t max_qubits, uint32_t* passes) {

@@ -86,6 +86,10 @@ int check_gate(uint64_t len, const qvnt_gate& g, bool* noop);
 int launch_gate(qvnt_reg* r, const qvnt_gate& g);
 int launch_init(qvnt_reg* r, uint64_t state);
 
+// runs.hip: a validated queue in the plain form: runs of SingleOps in one
+// pass each (runs.hpp), the others through launch_gate
+int apply_plain(qvnt_reg* r, const qvnt_gate* g, size_t n);
+
 // measure.hip
 int tree_build(qvnt_reg* r, uint64_t count, double* total_out);
 int tree_sample(qvnt_reg* r, uint64_t count, const double* u, size_t shots, uint64_t* out, double* total_out);

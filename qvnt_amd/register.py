@@ -187,7 +187,7 @@ class QReg:
         return lib.qvnt_reg_len(self._h)
 
     def apply(self, op):
-        """QReg::apply (quant.rs:376-395): one kernel per SingleOp, queue order."""
+        """QReg::apply (quant.rs:376-395): every SingleOp in queue order, with its own rounding."""
         if not isinstance(op, MultiOp):
             raise TypeError("apply expects a MultiOp")
         check(lib.qvnt_reg_apply(self._h, op.handle))
