@@ -3,11 +3,10 @@
 // The host compiler (fusion.cpp) turns the queue into passes; this kernel
 // runs one pass.  One block per tile of 2^t amplitudes (the tile's t qubits
 // are the pass's qubit set; blocks take tiles in XCD order, xcd_order).
-// The tile is read once from HBM, every phase
-// moves its 16 amplitudes per thread LDS -> registers -> LDS (skipped when
-// the phase's register qubits are the tile's top four, the layout of the
-// HBM access itself), and the tile is written back once.  HBM traffic is
-// one read and one write of the state per pass, whatever the number of
+// The tile is read once from HBM into registers, 16 amplitudes per thread,
+// moves through LDS from one phase's register layout to the next
+// (tile.hpp), and is written back once.  HBM traffic is one read and one
+// write of the state per pass, whatever the number of
 // gates in it.  Results agree with the plain form to rounding (FMA
 // contraction is on in this file; 2x2 products are merged on the host).
 #pragma clang fp contract(fast)
@@ -20,14 +19,22 @@
 #include "device.hpp"
 #include "fusion.hpp"
 #include "reg.hpp"
+#include "tile.hpp"
 
 namespace qvnt {
 namespace {
 
 using namespace fusion;
+using tile::exchange;
+using tile::layout_of;
+using tile::put;
+using tile::spread;
+using Layout = tile::Layout<kRegBits>;
+using tile::swz;
 
-// the LDS swizzle of fusion.hpp (lds_swizzle), for device code
-__device__ __forceinline__ uint32_t dswz(uint32_t e) { return e ^ ((e >> 4) & 15u); }
+// the local offset behind an offset of the program, which are swizzled as
+// fusion.hpp's lds_swizzle has it (its own inverse)
+__device__ __forceinline__ uint32_t unswizzled(uint32_t e) { return e ^ ((e >> 4) & 15u); }
 
 __device__ __forceinline__ double fmar(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fmar(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -48,27 +55,30 @@ __device__ __forceinline__ cplx<R> ld_coef(const double* __restrict__ c, int k) 
     return {(R)c[2 * k], (R)c[2 * k + 1]};
 }
 
-// 2x2 on register bit J for the register indices in the uniform pattern
-// pc (register controls); MASKED = false when there are none.
-template <int J, bool MASKED, class R>
-__device__ __forceinline__ void apply_m2(cplx<R>* v, const double* __restrict__ c, uint32_t pc) {
+// In the ops below M is false when the op acts on every register index and
+// every lane; otherwise pc is the uniform pattern of the register indices it
+// acts on and `on` says whether this lane does (controls on lane bits).
+
+// 2x2 on register bit J
+template <int J, bool M, class R>
+__device__ __forceinline__ void apply_m2(cplx<R>* v, const double* __restrict__ c, uint32_t pc, bool on) {
     const cplx<R> u00 = ld_coef<R>(c, 0), u01 = ld_coef<R>(c, 1), u10 = ld_coef<R>(c, 2), u11 = ld_coef<R>(c, 3);
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & (1 << J)) continue;
-        if (MASKED && !((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const cplx<R> x0 = v[i], x1 = v[i | (1 << J)];
-        v[i] = fma_c(mul_c(u00, x0), u01, x1);
-        v[i | (1 << J)] = fma_c(mul_c(u10, x0), u11, x1);
+        put<M>(v[i], fma_c(mul_c(u00, x0), u01, x1), on);
+        put<M>(v[i | (1 << J)], fma_c(mul_c(u10, x0), u11, x1), on);
     }
 }
 
-template <int J0, int J1, class R>
-__device__ __forceinline__ void apply_m4(cplx<R>* v, const double* __restrict__ c, uint32_t pc) {
+template <int J0, int J1, bool M, class R>
+__device__ __forceinline__ void apply_m4(cplx<R>* v, const double* __restrict__ c, uint32_t pc, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & ((1 << J0) | (1 << J1))) continue;
-        if (!((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const int idx[4] = {i, i | (1 << J0), i | (1 << J1), i | (1 << J0) | (1 << J1)};
         cplx<R> x[4];
 #pragma unroll
@@ -79,121 +89,111 @@ __device__ __forceinline__ void apply_m4(cplx<R>* v, const double* __restrict__ 
             acc = fma_c(acc, ld_coef<R>(c, 4 * r + 1), x[1]);
             acc = fma_c(acc, ld_coef<R>(c, 4 * r + 2), x[2]);
             acc = fma_c(acc, ld_coef<R>(c, 4 * r + 3), x[3]);
-            v[idx[r]] = acc;
+            put<M>(v[idx[r]], acc, on);
         }
     }
 }
 
 // anti-diagonal 2x2 (u00 = u11 = 0): out0 = u01 x1, out1 = u10 x0
-template <int J, bool MASKED, class R>
-__device__ __forceinline__ void apply_a2(cplx<R>* v, const double* __restrict__ c, uint32_t pc) {
+template <int J, bool M, class R>
+__device__ __forceinline__ void apply_a2(cplx<R>* v, const double* __restrict__ c, uint32_t pc, bool on) {
     const cplx<R> u01 = ld_coef<R>(c, 0), u10 = ld_coef<R>(c, 1);
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & (1 << J)) continue;
-        if (MASKED && !((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const cplx<R> x0 = v[i], x1 = v[i | (1 << J)];
-        v[i] = mul_c(u01, x1);
-        v[i | (1 << J)] = mul_c(u10, x0);
+        put<M>(v[i], mul_c(u01, x1), on);
+        put<M>(v[i | (1 << J)], mul_c(u10, x0), on);
     }
 }
 
 // the swap of the two halves (x, controlled x): no arithmetic
-template <int J, bool MASKED, class R>
-__device__ __forceinline__ void apply_x2(cplx<R>* v, uint32_t pc) {
+template <int J, bool M, class R>
+__device__ __forceinline__ void apply_x2(cplx<R>* v, uint32_t pc, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & (1 << J)) continue;
-        if (MASKED && !((pc >> i) & 1u)) continue;
-        const cplx<R> x0 = v[i];
-        v[i] = v[i | (1 << J)];
-        v[i | (1 << J)] = x0;
+        if (M && !((pc >> i) & 1u)) continue;
+        const cplx<R> x0 = v[i], x1 = v[i | (1 << J)];
+        put<M>(v[i], x1, on);
+        put<M>(v[i | (1 << J)], x0, on);
     }
 }
 
 // the real middle factor of a split 2x2 (fusion.hpp: OP_T2), one FMA per
 // real output: out0 = x0 - a x1, out1 = x1 + a x0
-template <int J, bool MASKED, class R>
-__device__ __forceinline__ void apply_t2(cplx<R>* v, R a, uint32_t pc) {
+template <int J, bool M, class R>
+__device__ __forceinline__ void apply_t2(cplx<R>* v, R a, uint32_t pc, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & (1 << J)) continue;
-        if (MASKED && !((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const cplx<R> x0 = v[i], x1 = v[i | (1 << J)];
-        v[i] = cplx<R>{fmar(-a, x1.re, x0.re), fmar(-a, x1.im, x0.im)};
-        v[i | (1 << J)] = cplx<R>{fmar(a, x0.re, x1.re), fmar(a, x0.im, x1.im)};
-    }
-}
-
-template <class R>
-__device__ __forceinline__ void apply_t2_sel(cplx<R>* v, R a, uint32_t sel, uint32_t pc) {
-    if (pc == 0xFFFFu) {
-        switch (sel) {
-        case 0: apply_t2<0, false>(v, a, 0u); break;
-        case 1: apply_t2<1, false>(v, a, 0u); break;
-        case 2: apply_t2<2, false>(v, a, 0u); break;
-        default: apply_t2<3, false>(v, a, 0u); break;
-        }
-    } else {
-        switch (sel) {
-        case 0: apply_t2<0, true>(v, a, pc); break;
-        case 1: apply_t2<1, true>(v, a, pc); break;
-        case 2: apply_t2<2, true>(v, a, pc); break;
-        default: apply_t2<3, true>(v, a, pc); break;
-        }
+        put<M>(v[i], cplx<R>{fmar(-a, x1.re, x0.re), fmar(-a, x1.im, x0.im)}, on);
+        put<M>(v[i | (1 << J)], cplx<R>{fmar(a, x0.re, x1.re), fmar(a, x0.im, x1.im)}, on);
     }
 }
 
 // 4x4 pairing r with r ^ 3 only: out[r] = u[r][r] x[r] + u[r][r^3] x[r^3]
-template <int J0, int J1, class R>
-__device__ __forceinline__ void apply_p4(cplx<R>* v, const double* __restrict__ c, uint32_t pc) {
+template <int J0, int J1, bool M, class R>
+__device__ __forceinline__ void apply_p4(cplx<R>* v, const double* __restrict__ c, uint32_t pc, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & ((1 << J0) | (1 << J1))) continue;
-        if (!((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const int idx[4] = {i, i | (1 << J0), i | (1 << J1), i | (1 << J0) | (1 << J1)};
-        cplx<R> x[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) x[k] = v[idx[k]];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            v[idx[r]] = fma_c(mul_c(ld_coef<R>(c, 2 * r), x[r]), ld_coef<R>(c, 2 * r + 1), x[r ^ 3]);
+        for (int r = 0; r < 2; ++r) {
+            const cplx<R> x = v[idx[r]], y = v[idx[r ^ 3]];
+            put<M>(v[idx[r]], fma_c(mul_c(ld_coef<R>(c, 2 * r), x), ld_coef<R>(c, 2 * r + 1), y), on);
+            put<M>(v[idx[r ^ 3]], fma_c(mul_c(ld_coef<R>(c, 2 * (r ^ 3)), y), ld_coef<R>(c, 2 * (r ^ 3) + 1), x), on);
+        }
     }
 }
 
 // P4 with real diagonal and imaginary pairing coefficients (fusion.hpp:
 // OP_P4R): out_r = c_r x_r + i s_r x_(r^3)
-template <int J0, int J1, class R>
-__device__ __forceinline__ void apply_p4r(cplx<R>* v, const double* __restrict__ c, uint32_t pc) {
+template <int J0, int J1, bool M, class R>
+__device__ __forceinline__ void apply_p4r(cplx<R>* v, const double* __restrict__ c, uint32_t pc, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
         if (i & ((1 << J0) | (1 << J1))) continue;
-        if (!((pc >> i) & 1u)) continue;
+        if (M && !((pc >> i) & 1u)) continue;
         const int idx[4] = {i, i | (1 << J0), i | (1 << J1), i | (1 << J0) | (1 << J1)};
-        cplx<R> x[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) x[k] = v[idx[k]];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const cplx<R> k = ld_coef<R>(c, r);
-            v[idx[r]] = cplx<R>{k.re * x[r].re - k.im * x[r ^ 3].im, k.re * x[r].im + k.im * x[r ^ 3].re};
+        for (int r = 0; r < 2; ++r) {
+            const cplx<R> x = v[idx[r]], y = v[idx[r ^ 3]];
+            const cplx<R> k = ld_coef<R>(c, r), q = ld_coef<R>(c, r ^ 3);
+            put<M>(v[idx[r]], cplx<R>{k.re * x.re - k.im * y.im, k.re * x.im + k.im * y.re}, on);
+            put<M>(v[idx[r ^ 3]], cplx<R>{q.re * y.re - q.im * x.im, q.re * y.im + q.im * x.re}, on);
         }
     }
 }
 
 // diagonal: one phase per register (host tables, controls folded in)
-template <class R>
-__device__ __forceinline__ void apply_d(cplx<R>* v, const double* __restrict__ c) {
+template <bool M, class R>
+__device__ __forceinline__ void apply_d(cplx<R>* v, const double* __restrict__ c, bool on) {
 #pragma unroll
-    for (int i = 0; i < kRegs; ++i) v[i] = mul_c(ld_coef<R>(c, i), v[i]);
+    for (int i = 0; i < kRegs; ++i) put<M>(v[i], mul_c(ld_coef<R>(c, i), v[i]), on);
+}
+// the same from a table of the lane's own: two phases loaded at a time, as
+// they take registers of every lane
+template <bool M, class R>
+__device__ __forceinline__ void apply_d_lane(cplx<R>* v, const double* __restrict__ c, bool on) {
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) {
+        put<M>(v[i], mul_c(ld_coef<R>(c, i), v[i]), on);
+        if (i & 1) asm volatile("" ::: "memory");
+    }
 }
 
 // a phase on the amplitudes whose register bit J is 1 (fusion.hpp: OP_PH)
-template <int J, class R>
-__device__ __forceinline__ void apply_ph(cplx<R>* v, const cplx<R> g) {
+template <int J, bool M, class R>
+__device__ __forceinline__ void apply_ph(cplx<R>* v, const cplx<R> g, bool on) {
 #pragma unroll
     for (int i = 0; i < kRegs; ++i)
-        if (i & (1 << J)) v[i] = mul_c(g, v[i]);
+        if (i & (1 << J)) put<M>(v[i], mul_c(g, v[i]), on);
 }
 
 // the structured block (fusion.hpp: OP_S): diagonal, T2 on register bits
@@ -202,14 +202,13 @@ __device__ __forceinline__ void apply_ph(cplx<R>* v, const cplx<R> g) {
 // from the first product to the last
 template <bool D1, bool D2, class R>
 __device__ __forceinline__ void apply_s(cplx<R>* v, const double* __restrict__ c) {
-    if (D1) apply_d(v, c);
-    apply_t2<0, false>(v, (R)c[2 * kRegs + 0], 0u);
-    apply_t2<1, false>(v, (R)c[2 * kRegs + 2], 0u);
-    apply_t2<2, false>(v, (R)c[2 * kRegs + 4], 0u);
-    apply_t2<3, false>(v, (R)c[2 * kRegs + 6], 0u);
-    if (D2) apply_d(v, c + 2 * (kRegs + kRegBits));
+    if (D1) apply_d<false>(v, c, true);
+    apply_t2<0, false>(v, (R)c[2 * kRegs + 0], 0u, true);
+    apply_t2<1, false>(v, (R)c[2 * kRegs + 2], 0u, true);
+    apply_t2<2, false>(v, (R)c[2 * kRegs + 4], 0u, true);
+    apply_t2<3, false>(v, (R)c[2 * kRegs + 6], 0u, true);
+    if (D2) apply_d<false>(v, c + 2 * (kRegs + kRegBits), true);
 }
-
 
 // T2's and PH's coefficient, carried in the op (fusion.hpp: FOp::ga, gb)
 template <class R>
@@ -217,138 +216,151 @@ __device__ __forceinline__ cplx<R> inline_coef(const FOp& op) {
     return cplx<R>{(R)__longlong_as_double((long long)op.ga), (R)__longlong_as_double((long long)op.gb)};
 }
 
+// over the active lanes of the wave; uniform
+__device__ __forceinline__ bool some(bool x) { return __builtin_amdgcn_ballot_w64(x) != 0; }
+__device__ __forceinline__ bool every(bool x) { return __builtin_amdgcn_ballot_w64(!x) == 0; }
+
+// One op other than G, S and D.
+template <bool M, class R>
+__device__ __forceinline__ void apply_op(cplx<R>* v, const FOp& op, const double* __restrict__ c, bool on) {
+    switch (op.type) {
+    case OP_PH:
+        switch (op.sel) {
+        case 0: apply_ph<0, M>(v, inline_coef<R>(op), on); break;
+        case 1: apply_ph<1, M>(v, inline_coef<R>(op), on); break;
+        case 2: apply_ph<2, M>(v, inline_coef<R>(op), on); break;
+        default: apply_ph<3, M>(v, inline_coef<R>(op), on); break;
+        }
+        break;
+    case OP_T2:
+        switch (op.sel) {
+        case 0: apply_t2<0, M>(v, inline_coef<R>(op).re, op.pc, on); break;
+        case 1: apply_t2<1, M>(v, inline_coef<R>(op).re, op.pc, on); break;
+        case 2: apply_t2<2, M>(v, inline_coef<R>(op).re, op.pc, on); break;
+        default: apply_t2<3, M>(v, inline_coef<R>(op).re, op.pc, on); break;
+        }
+        break;
+    case OP_M2:
+        switch (op.sel) {
+        case 0: apply_m2<0, M>(v, c, op.pc, on); break;
+        case 1: apply_m2<1, M>(v, c, op.pc, on); break;
+        case 2: apply_m2<2, M>(v, c, op.pc, on); break;
+        default: apply_m2<3, M>(v, c, op.pc, on); break;
+        }
+        break;
+    case OP_M4:
+        switch (op.sel) {
+        case 1: apply_m4<0, 1, M>(v, c, op.pc, on); break;
+        case 2: apply_m4<0, 2, M>(v, c, op.pc, on); break;
+        case 3: apply_m4<0, 3, M>(v, c, op.pc, on); break;
+        case 6: apply_m4<1, 2, M>(v, c, op.pc, on); break;
+        case 7: apply_m4<1, 3, M>(v, c, op.pc, on); break;
+        default: apply_m4<2, 3, M>(v, c, op.pc, on); break;
+        }
+        break;
+    case OP_P4:
+        switch (op.sel) {
+        case 1: apply_p4<0, 1, M>(v, c, op.pc, on); break;
+        case 2: apply_p4<0, 2, M>(v, c, op.pc, on); break;
+        case 3: apply_p4<0, 3, M>(v, c, op.pc, on); break;
+        case 6: apply_p4<1, 2, M>(v, c, op.pc, on); break;
+        case 7: apply_p4<1, 3, M>(v, c, op.pc, on); break;
+        default: apply_p4<2, 3, M>(v, c, op.pc, on); break;
+        }
+        break;
+    case OP_P4R:
+        switch (op.sel) {
+        case 1: apply_p4r<0, 1, M>(v, c, op.pc, on); break;
+        case 2: apply_p4r<0, 2, M>(v, c, op.pc, on); break;
+        case 3: apply_p4r<0, 3, M>(v, c, op.pc, on); break;
+        case 6: apply_p4r<1, 2, M>(v, c, op.pc, on); break;
+        case 7: apply_p4r<1, 3, M>(v, c, op.pc, on); break;
+        default: apply_p4r<2, 3, M>(v, c, op.pc, on); break;
+        }
+        break;
+    case OP_A2:
+        switch (op.sel) {
+        case 0: apply_a2<0, M>(v, c, op.pc, on); break;
+        case 1: apply_a2<1, M>(v, c, op.pc, on); break;
+        case 2: apply_a2<2, M>(v, c, op.pc, on); break;
+        default: apply_a2<3, M>(v, c, op.pc, on); break;
+        }
+        break;
+    default:
+        switch (op.sel) {
+        case 0: apply_x2<0, M>(v, op.pc, on); break;
+        case 1: apply_x2<1, M>(v, op.pc, on); break;
+        case 2: apply_x2<2, M>(v, op.pc, on); break;
+        default: apply_x2<3, M>(v, op.pc, on); break;
+        }
+        break;
+    }
+}
+
+// No branch in here diverges: a wave whose lanes all satisfy an op's lane
+// controls runs it whole, one with none skips it, a mixed one selects per
+// lane.  (A divergent branch around the op makes the compiler keep the 16
+// amplitudes twice, old and new: 221 VGPRs in FP64.)
 template <class R>
 __device__ __forceinline__ void run_phase(cplx<R>* v, const FPhase& ph, const FOp* __restrict__ ops,
                                           const double* __restrict__ coef, uint32_t tb, uint64_t tile) {
     // the product of the phase's G factors (uniform, accumulated in FP64)
     cplx<double> scal{1.0, 0.0};
     bool scaled = false;
-    // Each op's header is loaded when the op starts.  Loading the next one
-    // ahead held 16 more SGPRs through the op body and doubled the SGPR
-    // spills (into VGPR lanes); the whole-circuit passes ran 3% slower.
-    for (uint32_t o = ph.op_begin; o < ph.op_end; ++o) {
-        const FOp op = ops[o];
-        // controls on lane bits (this thread's base) and on bits outside the tile
-        if ((tb & op.lctrl) != op.lctrl || (tile & op.gctrl) != op.gctrl) continue;
+    const uint32_t end = ph.op_end;
+    for (uint32_t o = ph.op_begin; o < end; ++o) {
+        const FOp& op = ops[o];
+        // controls on lane bits (this thread's base) and on bits outside the
+        // tile (which differ between the lanes of a wave only where it holds
+        // several small tiles, see persist_unit)
+        const bool on = (tb & op.lctrl) == op.lctrl && (tile & op.gctrl) == op.gctrl;
+        if (!some(on)) continue;
+        const bool all = every(on);
         const double* c = coef + op.coef;
-        if (op.type == OP_G) {
-            const uint32_t k = ((tile & op.ga) != 0 ? 1u : 0u) | ((tile & op.gb) != 0 ? 2u : 0u);
-            scal = mul_c(ld_coef<double>(c, (int)(k * kRegs)), scal);
-            scaled = true;
-        } else if (op.type == OP_D) {
-            // table variant from the non-register operands (uniform branches)
-            const bool ea = (op.la | op.ga) != 0, eb = (op.lb | op.gb) != 0;
-            const uint32_t k = ((((tb & op.la) | (tile & op.ga)) != 0) ? 1u : 0u) |
-                               ((((tb & op.lb) | (tile & op.gb)) != 0) ? 2u : 0u);
-            // dmode 1: the variant-0 table, then (waves whose operand bit is
-            // set) the ratio table, both uniform loads; else each lane loads
-            // its own variant
-            if (!ea && !eb) {
-                apply_d(v, c);
-            } else if (op.dmode == 1) {
-                apply_d(v, c);
-                const uint32_t var = ea ? 1u : 2u;
-                if (k & var) apply_d(v, c + 2 * kRegs * var);  // uniform branch
-            } else {
-                apply_d(v, c + 2 * kRegs * k);  // per-lane variant table
-            }
-        } else if (op.type == OP_S) {
+        const uint32_t type = op.type;
+        if (type == OP_S) {
             switch (op.sel) {
             case 0: apply_s<false, false>(v, c); break;
             case 1: apply_s<true, false>(v, c); break;
             case 2: apply_s<false, true>(v, c); break;
             default: apply_s<true, true>(v, c); break;
             }
-        } else if (op.type == OP_PH) {
-            switch (op.sel) {
-            case 0: apply_ph<0>(v, inline_coef<R>(op)); break;
-            case 1: apply_ph<1>(v, inline_coef<R>(op)); break;
-            case 2: apply_ph<2>(v, inline_coef<R>(op)); break;
-            default: apply_ph<3>(v, inline_coef<R>(op)); break;
-            }
-        } else if (op.type == OP_T2) {
-            apply_t2_sel(v, inline_coef<R>(op).re, op.sel, op.pc);
-        } else if (op.type == OP_M2) {
-            if (op.pc == 0xFFFFu) {
-                switch (op.sel) {
-                case 0: apply_m2<0, false>(v, c, 0u); break;
-                case 1: apply_m2<1, false>(v, c, 0u); break;
-                case 2: apply_m2<2, false>(v, c, 0u); break;
-                default: apply_m2<3, false>(v, c, 0u); break;
-                }
+        } else if (type == OP_G) {
+            const uint32_t k = ((tile & op.ga) != 0 ? 1u : 0u) | ((tile & op.gb) != 0 ? 2u : 0u);
+            const cplx<double> g = mul_c(ld_coef<double>(c, (int)(k * kRegs)), scal);
+            scal.re = on ? g.re : scal.re;
+            scal.im = on ? g.im : scal.im;
+            scaled |= on;
+        } else if (type == OP_D) {
+            // table variant from the non-register operands
+            const bool ea = (op.la | op.ga) != 0, eb = (op.lb | op.gb) != 0;
+            const uint32_t k = ((((tb & op.la) | (tile & op.ga)) != 0) ? 1u : 0u) |
+                               ((((tb & op.lb) | (tile & op.gb)) != 0) ? 2u : 0u);
+            // dmode 1: the variant-0 table, then (waves whose operand bit is
+            // set) the ratio table, both uniform loads; else each lane loads
+            // its own variant
+            if ((ea || eb) && op.dmode != 1) {
+                apply_d_lane<true>(v, c + 2 * kRegs * k, on);
             } else {
-                switch (op.sel) {
-                case 0: apply_m2<0, true>(v, c, op.pc); break;
-                case 1: apply_m2<1, true>(v, c, op.pc); break;
-                case 2: apply_m2<2, true>(v, c, op.pc); break;
-                default: apply_m2<3, true>(v, c, op.pc); break;
+                const uint32_t var = ea ? 1u : 2u;
+                if (all) apply_d<false>(v, c, true);
+                else apply_d<true>(v, c, on);
+                const bool second = (ea || eb) && (k & var) != 0 && on;
+                if (some(second)) {
+                    if (every(second)) apply_d<false>(v, c + 2 * kRegs * var, true);
+                    else apply_d<true>(v, c + 2 * kRegs * var, second);
                 }
             }
-        } else if (op.type == OP_M4) {
-            switch (op.sel) {
-            case 1: apply_m4<0, 1>(v, c, op.pc); break;
-            case 2: apply_m4<0, 2>(v, c, op.pc); break;
-            case 3: apply_m4<0, 3>(v, c, op.pc); break;
-            case 6: apply_m4<1, 2>(v, c, op.pc); break;
-            case 7: apply_m4<1, 3>(v, c, op.pc); break;
-            default: apply_m4<2, 3>(v, c, op.pc); break;
-            }
-        } else if (op.type == OP_P4) {
-            switch (op.sel) {
-            case 1: apply_p4<0, 1>(v, c, op.pc); break;
-            case 2: apply_p4<0, 2>(v, c, op.pc); break;
-            case 3: apply_p4<0, 3>(v, c, op.pc); break;
-            case 6: apply_p4<1, 2>(v, c, op.pc); break;
-            case 7: apply_p4<1, 3>(v, c, op.pc); break;
-            default: apply_p4<2, 3>(v, c, op.pc); break;
-            }
-        } else if (op.type == OP_P4R) {
-            switch (op.sel) {
-            case 1: apply_p4r<0, 1>(v, c, op.pc); break;
-            case 2: apply_p4r<0, 2>(v, c, op.pc); break;
-            case 3: apply_p4r<0, 3>(v, c, op.pc); break;
-            case 6: apply_p4r<1, 2>(v, c, op.pc); break;
-            case 7: apply_p4r<1, 3>(v, c, op.pc); break;
-            default: apply_p4r<2, 3>(v, c, op.pc); break;
-            }
-        } else if (op.type == OP_A2) {
-            if (op.pc == 0xFFFFu) {
-                switch (op.sel) {
-                case 0: apply_a2<0, false>(v, c, 0u); break;
-                case 1: apply_a2<1, false>(v, c, 0u); break;
-                case 2: apply_a2<2, false>(v, c, 0u); break;
-                default: apply_a2<3, false>(v, c, 0u); break;
-                }
-            } else {
-                switch (op.sel) {
-                case 0: apply_a2<0, true>(v, c, op.pc); break;
-                case 1: apply_a2<1, true>(v, c, op.pc); break;
-                case 2: apply_a2<2, true>(v, c, op.pc); break;
-                default: apply_a2<3, true>(v, c, op.pc); break;
-                }
-            }
+        } else if (all && op.pc == 0xFFFFu) {
+            apply_op<false>(v, op, c, true);
         } else {
-            if (op.pc == 0xFFFFu) {
-                switch (op.sel) {
-                case 0: apply_x2<0, false>(v, 0u); break;
-                case 1: apply_x2<1, false>(v, 0u); break;
-                case 2: apply_x2<2, false>(v, 0u); break;
-                default: apply_x2<3, false>(v, 0u); break;
-                }
-            } else {
-                switch (op.sel) {
-                case 0: apply_x2<0, true>(v, op.pc); break;
-                case 1: apply_x2<1, true>(v, op.pc); break;
-                case 2: apply_x2<2, true>(v, op.pc); break;
-                default: apply_x2<3, true>(v, op.pc); break;
-                }
-            }
+            apply_op<true>(v, op, c, on);
         }
     }
-    if (scaled) {
+    if (some(scaled)) {
         const cplx<R> f{(R)scal.re, (R)scal.im};
 #pragma unroll
-        for (int i = 0; i < kRegs; ++i) v[i] = mul_c(f, v[i]);
+        for (int i = 0; i < kRegs; ++i) put<true>(v[i], mul_c(f, v[i]), scaled);
     }
 }
 
@@ -369,60 +381,56 @@ template <class R> struct AccOf;
 template <> struct AccOf<double> { typedef mf64x4 type; static constexpr bool hi_low_bits = true; };
 template <> struct AccOf<float> { typedef mf32x4 type; static constexpr bool hi_low_bits = false; };
 
-// swizzled LDS offset of register-index bits (j & 3) placed at register
-// bits (b0, b0 + 1) of the phase: the swizzle is XOR-linear, so offsets of
-// disjoint bit groups combine by XOR
-__device__ __forceinline__ uint32_t reg_off2(const FPhase& ph, int b0, uint32_t j) {
-    return dswz(((j & 1u) << ph.rpos[b0]) | (((j >> 1) & 1u) << ph.rpos[b0 + 1]));
+// The register layout of a dense phase (16x16 unitary U on the phase's
+// register bits): the tile is a 16 x 2^(t-4) complex matrix X, row = register
+// index of the phase, column = thread base, and each 64-lane wave owns the 64
+// columns of its own threads.  Lane l holds, in register 4 c + s, the element
+// of row 4 s + l / 16 and column 16 c + l % 16 of them: the matrix cores'
+// B operand of step s for column tile c.
+__device__ __forceinline__ Layout dense_layout(const FPhase& ph, uint32_t tid) {
+    const uint32_t hi = (tid >> 4) & 3u;
+    uint32_t e = spread<kRegBits>(tid & ~48u, ph.rpos);
+    e |= ((hi & 1u) << ph.rpos[0]) | ((hi >> 1) << ph.rpos[1]);
+    Layout l;
+    l.base = swz(e);
+    l.bit[0] = swz(1u << ph.rpos[2]);
+    l.bit[1] = swz(1u << ph.rpos[3]);
+    l.bit[2] = swz(spread<kRegBits>(16u, ph.rpos));
+    l.bit[3] = swz(spread<kRegBits>(32u, ph.rpos));
+    return l;
 }
 
-// A dense phase: the tile (in LDS) is a 16 x 2^(t-4) complex matrix X
-// (row = register index of the phase, column = thread base), and the phase
-// computes X := U X as a real 32x32 GEMM on the matrix cores:
+// X := U X in dense_layout, as a real 32x32 GEMM on the matrix cores:
 //   Yre = Ure Xre - Uim Xim,   Yim = Ure Xim + Uim Xre.
-// Each 64-lane wave owns the 64 columns of its own threads (as in the
-// register phases), in four 16-column tiles; all reads of a tile's columns
-// precede its writes, so the update is in place.
+// The result comes out in the layout it went in: element i of lane l's
+// accumulator is row l / 16 + 4 i in f64, and in f32, where it is row
+// 4 (l / 16) + i, U's rows are taken in the order that makes it so.
 template <class R>
-__device__ __forceinline__ void dense_phase(cplx<R>* lds, const FPhase& ph, const double* __restrict__ u, uint32_t tid) {
+__device__ __forceinline__ void dense_phase(cplx<R>* v, const double* __restrict__ u, uint32_t tid) {
     typedef typename AccOf<R>::type Acc;
-    const uint32_t lane = tid & 63u, hi = lane >> 4, wave0 = tid & ~63u;
-    // A operands: U[m][4s + hi] with m = lane % 16
-    R ure[4], uim[4], nuim[4];
+    const uint32_t lane = tid & 63u, hi = lane >> 4, m = lane & 15u;
+    // A operands: row m (f32: of the reordered U) and column 4 s + hi
+    const uint32_t row = AccOf<R>::hi_low_bits ? m : (m >> 2) | ((m & 3u) << 2);
+    R ure[4], uim[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const int e = 16 * (int)(lane & 15u) + 4 * s + (int)hi;
+        const uint32_t e = 16u * row + 4u * (uint32_t)s + hi;
         ure[s] = (R)u[2 * e];
         uim[s] = (R)u[2 * e + 1];
-        nuim[s] = -uim[s];
     }
-    const uint32_t in_hi = reg_off2(ph, 0, hi);   // B rows 4s + hi: register bits 0,1 = hi
-    // accumulator rows: hi + 4i (f64) or 4 hi + i (f32)
-    constexpr bool lowhi = AccOf<R>::hi_low_bits;
-    const uint32_t out_hi = reg_off2(ph, lowhi ? 0 : 2, hi);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        // this lane's column and its LDS base (zeros at the register bits)
-        uint32_t tb = wave0 + 16u * c + (lane & 15u);
-#pragma unroll
-        for (int k = 0; k < kRegBits; ++k) {
-            const uint32_t lo = tb & ((1u << ph.rpos[k]) - 1u);
-            tb = ((tb ^ lo) << 1) | lo;
-        }
-        const uint32_t stb = dswz(tb);
-        cplx<R> x[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) x[s] = lds[stb ^ in_hi ^ reg_off2(ph, 2, (uint32_t)s)];
         Acc yre = {0, 0, 0, 0}, yim = {0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            yre = mfma(ure[s], x[s].re, yre);
-            yim = mfma(ure[s], x[s].im, yim);
-            yre = mfma(nuim[s], x[s].im, yre);
-            yim = mfma(uim[s], x[s].re, yim);
+            const cplx<R> x = v[4 * c + s];
+            yre = mfma(ure[s], x.re, yre);
+            yim = mfma(ure[s], x.im, yim);
+            yre = mfma(-uim[s], x.im, yre);
+            yim = mfma(uim[s], x.re, yim);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) lds[stb ^ out_hi ^ reg_off2(ph, lowhi ? 2 : 0, (uint32_t)i)] = cplx<R>{yre[i], yim[i]};
+        for (int i = 0; i < 4; ++i) put<false>(v[4 * c + i], cplx<R>{yre[i], yim[i]}, true);
     }
 }
 
@@ -452,153 +460,158 @@ __device__ __forceinline__ void load_tpos(const FPass& pass, uint32_t* tp) {
     for (int k = 0; k < kMaxTile; ++k) tp[k] = (w[k / 4] >> (8 * (k % 4))) & 63u;
 }
 
-// This thread's swizzled LDS offset in the direct layout, made opaque at
-// its use: the 16 offsets derived from it are used at most twice per tile,
-// and keeping them live across the phases (where the compiler would hoist
-// them) costs 16 VGPRs for the whole kernel.
-__device__ __forceinline__ uint32_t direct_base(uint32_t tid) {
-    uint32_t s = dswz(tid);
-    asm volatile("" : "+v"(s));
-    return s;
+// global offset of local index l (bits from t up are zero)
+__device__ __forceinline__ uint64_t global_offset(const uint32_t* tp, uint32_t l) {
+    uint64_t off = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxTile; ++k) off |= (uint64_t)((l >> k) & 1u) << tp[k];
+    return off;
 }
 
-// The tile's final read-out from LDS into the direct layout (register j =
-// local tid + j * nth), through the pass's qubit permutation if it has one.
-// KARG: the pass is a kernel argument (k_fused): its tables are read bit by
-// bit, in a loop -- fully unrolled, the compiler hoists those loads to the
-// kernel's start and the extra live scalar registers spill.  Passes in
-// global memory (the batched kernels) take the unrolled form: one wide
-// scalar load instead of a dependent load per bit.
-template <class R, bool KARG>
-__device__ __forceinline__ void read_out(cplx<R>* v, const cplx<R>* lds, const FPass& pass, uint32_t tid) {
-    if (pass.permuted) {
-        uint32_t s = 0;
-        if (KARG) {
-            for (uint32_t k = 0; k + kRegBits < pass.t; ++k)
-                if (tid >> k & 1) s ^= pass.pimg[k];
-        } else {
-            // (tid's bits from t-4 up and pimg's entries there are zero)
-#pragma unroll
-            for (uint32_t k = 0; k < (uint32_t)(kMaxTile - kRegBits); ++k) s ^= pass.pimg[k] & (0u - ((tid >> k) & 1u));
-        }
-#pragma unroll
-        for (int j = 0; j < kRegs; ++j) v[j] = lds[s ^ pass.pout[j]];
-    } else {
-        const uint32_t nth = pass.nthreads;
-#pragma unroll
-        for (int j = 0, sdir = direct_base(tid); j < kRegs; ++j) v[j] = lds[sdir ^ dswz(j * nth)];
-    }
-}
-
-// The phases of one pass on one tile.  On entry and on exit v holds the
-// thread's amplitudes in the direct layout (register j = local tid + j *
-// nth); `lds` is the tile's swizzled LDS copy (local element e at dswz(e)).
-template <class R, bool KARG>
-__device__ __forceinline__ void tile_phases(cplx<R>* v, cplx<R>* lds, const FPass& pass, const FPhase* __restrict__ phases,
-                                            const FOp* __restrict__ ops, const double* __restrict__ coef, uint64_t tile,
-                                            uint32_t tid) {
-    const uint32_t nth = pass.nthreads;
-    const uint32_t p0 = pass.phase_begin, p1 = pass.phase_end;
-    for (uint32_t p = p0; p < p1; ++p) {
-        const FPhase& ph = phases[p];
-        if (ph.dense) {
-            // works on the LDS tile: bring the HBM registers in first, and
-            // take the result back out for the final store
-            if (p == p0) {
-#pragma unroll
-                for (int j = 0, sdir = direct_base(tid); j < kRegs; ++j) lds[sdir ^ dswz(j * nth)] = v[j];
-                __syncthreads();
-            }
-            dense_phase<R>(lds, ph, coef + ph.ucoef, tid);
-            __syncthreads();
-            if (p + 1 == p1) read_out<R, KARG>(v, lds, pass, tid);
-            continue;
-        }
-        // local base of this thread in the phase: zeros at the register bits
-        uint32_t tb = tid;
-#pragma unroll
-        for (int k = 0; k < kRegBits; ++k) {
-            const uint32_t lo = tb & ((1u << ph.rpos[k]) - 1u);
-            tb = ((tb ^ lo) << 1) | lo;
-        }
-        const uint32_t stb = dswz(tb);
-        const bool direct_in = (p == p0) && pass.direct_first;
-        const bool direct_out = (p + 1 == p1) && pass.direct_last;
-        if (!direct_in) {
-            if (p == p0) {
-#pragma unroll
-                for (int j = 0, sdir = direct_base(tid); j < kRegs; ++j) lds[sdir ^ dswz(j * nth)] = v[j];
-                __syncthreads();
-            }
-#pragma unroll
-            for (int i = 0; i < kRegs; ++i) v[i] = lds[stb ^ ph.sroff[i]];
-        }
-        run_phase(v, ph, ops, coef, tb, tile);
-        if (!direct_out) {
-#pragma unroll
-            for (int i = 0; i < kRegs; ++i) lds[stb ^ ph.sroff[i]] = v[i];
-            __syncthreads();
-            if (p + 1 == p1) read_out<R, KARG>(v, lds, pass, tid);
-        }
-    }
-}
-
-// global offset of this thread's local bits 0..t-5
-__device__ __forceinline__ uint64_t thread_offset(const uint32_t* tp, uint32_t tid) {
-    uint64_t lo_off = 0;
-    // tid < 2^(t-4): its bits from t-4 up are zero
-#pragma unroll
-    for (uint32_t k = 0; k < (uint32_t)(kMaxTile - kRegBits); ++k) lo_off |= (uint64_t)((tid >> k) & 1u) << tp[k];
-    return lo_off;
-}
-// every amplitude of the tile is read once and written once per pass:
-// non-temporal stores (streamed through the caches, evicted first)
+// Where the tile is read from or written to HBM: the local bits the
+// registers run over, and the thread's address.
 template <class R>
-__device__ __forceinline__ void store_direct(cplx<R>* __restrict__ psi, const FPass& pass, uint64_t base, const cplx<R>* v) {
+struct Edge {
+    uint32_t pos[kRegBits];
+    uint32_t tb;              // local index of register 0
+    uint64_t step[kRegBits];  // global offsets of the register bits (uniform)
+    // own: in the layout of phase ph, else with the tile's top bits in the registers
+    __device__ __forceinline__ void set(const FPass& pass, const FPhase& ph, bool own, uint32_t tid) {
 #pragma unroll
-    for (int j = 0; j < kRegs; ++j) {
-        cplx<R>* p = psi + base + pass.hoff[j];
-        __builtin_nontemporal_store(v[j].re, &p->re);
-        __builtin_nontemporal_store(v[j].im, &p->im);
+        for (int j = 0; j < kRegBits; ++j) {
+            pos[j] = own ? ph.rpos[j] : pass.t - kRegBits + j;
+            step[j] = 1ull << pass.tpos[pos[j]];
+        }
+        tb = spread<kRegBits>(tid, pos);
     }
+    __device__ __forceinline__ uint64_t off(int i) const {
+        uint64_t o = 0;
+#pragma unroll
+        for (int j = 0; j < kRegBits; ++j)
+            if (i >> j & 1) o |= step[j];
+        return o;
+    }
+};
+
+// Whether a tile can be read or written in the phase's own layout: a whole
+// 128-byte line has to stay among the threads (local bits 0..2 in FP64, 0..3
+// in FP32).  Saves one exchange.
+template <class R>
+__device__ __forceinline__ bool edge_layout(const FPhase& ph) {
+    return !ph.dense && ph.rpos[0] >= (sizeof(R) == 8 ? 3u : 4u);
+}
+
+// Passes of at most this many tiles bring their program near first
+// (warm_program).  With more, the blocks before have done so, and the touches
+// only take time: 31-qubit Ising steps in FP32 96 ms without, 112 with.
+constexpr uint32_t kWarmTiles = 2048;
+
+// Brings the pass's ops and coefficients into the L2 of this block's XCD:
+// thread k touches op k and its coefficient lines, all at once, where the op
+// loop's scalar loads would wait for memory one after the other (16 qubits
+// FP64, 400 gates: 370 us of k_fused without, 250 with).
+__device__ __forceinline__ uint32_t warm_program(const FOp* __restrict__ ops, const double* __restrict__ coef, uint32_t begin,
+                                                 uint32_t end, uint32_t tid, uint32_t nth) {
+    uint32_t seen = 0;
+    for (uint32_t o = begin + tid; o < end; o += nth) {
+        const FOp& op = ops[o];
+        const uint32_t type = op.type, c = op.coef;
+        const bool outside = ((uint64_t)(op.la | op.lb) | op.ga | op.gb) != 0;
+        const uint32_t n = type == OP_S ? 72u : type == OP_G ? 128u : type == OP_D ? (outside ? 128u : 32u) : type == OP_M4 ? 32u : type == OP_P4 ? 16u
+                           : type == OP_M2 || type == OP_P4R ? 8u : type == OP_A2 ? 4u : 0u;
+        for (uint32_t k = 0; k < n; k += 16u) seen ^= reinterpret_cast<const uint32_t*>(coef + c + k)[0];
+    }
+    return seen;
 }
 
 // One tile of one pass: read 2^t amplitudes, run the pass's phases, write
 // them back; the pass and program live in scalar-loadable memory.
-// tid: the thread's index within the tile (0 .. 2^(t-4) - 1).  ACTIVE
-// false: the threads run the phases (and their barriers) on their own LDS
-// region but neither read nor write HBM -- a block of the persistent
-// batched kernel whose tile group has no tile (see k_batch_persist).
-template <class R, bool KARG, bool GATED = false>
+// tiles: of the pass (kWarmTiles); tid: the thread's index within the tile (0 .. 2^(t-4) - 1); lds: 2^t
+// reals.  ACTIVE false: the threads run the phases (and their barriers) on
+// their own LDS region but neither read nor write HBM -- a block of the
+// persistent batched kernel whose tile group has no tile (see
+// k_batch_persist).
+template <class R, bool GATED = false>
 __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPass& pass, const FPhase* __restrict__ phases,
                                            const FOp* __restrict__ ops, const double* __restrict__ coef,
-                                           uint64_t tile_index, cplx<R>* lds, uint32_t tid, bool active = true) {
+                                           uint64_t tile_index, uint32_t tiles, R* lds, uint32_t tid, bool active = true) {
     uint32_t tp[kMaxTile];
     load_tpos(pass, tp);
     const uint64_t tile = tile_base(tp, pass.t, tile_index);
-    const uint64_t base = tile | thread_offset(tp, tid);
+    const uint32_t p0 = pass.phase_begin, p1 = pass.phase_end;
     cplx<R> v[kRegs];
+    const bool own_in = edge_layout<R>(phases[p0]);
+    uint32_t tb;
+    Layout cur;
+    {
+        Edge<R> in;
+        in.set(pass, phases[p0], own_in, tid);
+        tb = in.tb;
+        cur = layout_of<kRegBits>(tb, in.pos);
+        const cplx<R>* p = psi + (tile | global_offset(tp, tb));
 #pragma unroll
-    for (int j = 0; j < kRegs; ++j) {
-        v[j] = cplx<R>{(R)0, (R)0};
-        if (!GATED || active) {
-            const cplx<R>* p = psi + base + pass.hoff[j];
-            v[j] = cplx<R>{__builtin_nontemporal_load(&p->re), __builtin_nontemporal_load(&p->im)};
+        for (int i = 0; i < kRegs; ++i) {
+            v[i] = cplx<R>{(R)0, (R)0};
+            if (!GATED || active) {
+                const cplx<R>* q = p + in.off(i);
+                v[i] = cplx<R>{__builtin_nontemporal_load(&q->re), __builtin_nontemporal_load(&q->im)};
+            }
         }
     }
-    tile_phases<R, KARG>(v, lds, pass, phases, ops, coef, tile, tid);
-    if (!GATED || active) store_direct(psi, pass, base, v);
+    if (tiles <= kWarmTiles) {
+        const uint32_t seen = warm_program(ops, coef, phases[p0].op_begin, phases[p1 - 1].op_end, tid, pass.nthreads);
+        asm volatile("" ::"v"(seen));
+    }
+    for (uint32_t p = p0; p < p1; ++p) {
+        const FPhase& ph = phases[p];
+        if (ph.dense) {
+            const Layout to = dense_layout(ph, tid);
+            exchange<kRegBits>(v, lds, cur, to);
+            cur = to;
+            dense_phase(v, coef + ph.ucoef, tid);
+            continue;
+        }
+        if (p != p0 || !(own_in || pass.direct_first)) {
+            tb = spread<kRegBits>(tid, ph.rpos);
+            const Layout to = layout_of<kRegBits>(tb, ph.rpos);
+            exchange<kRegBits>(v, lds, cur, to);
+            cur = to;
+        }
+        run_phase(v, ph, ops, coef, tb, tile);
+    }
+    const FPhase& last = phases[p1 - 1];
+    const bool own_out = edge_layout<R>(last) && !pass.permuted;
+    Edge<R> out;
+    out.set(pass, last, own_out, tid);
+    if (pass.permuted) {
+        // through the pass's qubit permutation: the thread that stores local
+        // index tid + j 2^(t-4) reads it from pimg / pout
+        uint32_t s = 0;
+        for (uint32_t k = 0; k + kRegBits < pass.t; ++k) s ^= unswizzled(pass.pimg[k]) & (0u - ((tid >> k) & 1u));
+        s = swz(s);
+        exchange<kRegBits>(v, lds, cur, [&](int i) { return s ^ swz(unswizzled(pass.pout[i])); });
+    } else if (!own_out && !pass.direct_last) {
+        exchange<kRegBits>(v, lds, cur, layout_of<kRegBits>(out.tb, out.pos));
+    }
+    if (!GATED || active) {
+        // every amplitude of the tile is read once and written once per
+        // pass: non-temporal stores (streamed through the caches, evicted first)
+        cplx<R>* p = psi + (tile | global_offset(tp, out.tb));
+#pragma unroll
+        for (int i = 0; i < kRegs; ++i) {
+            cplx<R>* q = p + out.off(i);
+            __builtin_nontemporal_store(v[i].re, &q->re);
+            __builtin_nontemporal_store(v[i].im, &q->im);
+        }
+    }
 }
 
-// At most two waves per SIMD: the 64 KiB LDS tile allows no more, and the
-// whole VGPR file then holds the 16 amplitudes and the op operands
-// without spills.  (QVNT_FUSED_WAVES, a build-time knob, asks for that many
-// waves per SIMD instead: the VGPR budget shrinks to 512 / waves.)
-#ifdef QVNT_FUSED_WAVES
-#define QVNT_FUSED_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(QVNT_FUSED_WAVES, QVNT_FUSED_WAVES)))
-#else
-#define QVNT_FUSED_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2)))
-#endif
+// Four waves per SIMD: the exchange takes half a tile of LDS (32 KiB for
+// 2^12 FP64 or 2^13 FP32 amplitudes), and the op code keeps one copy of the
+// 16 amplitudes.  The persistent kernel's loop state does not fit beside
+// them in 128 registers: three.
+#define QVNT_FUSED_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
+#define QVNT_PERSIST_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 3)))
 
 // XCD-aware block order.  The dispatcher hands workgroups to the eight XCDs
 // round robin (block b to XCD b mod 8), and each XCD has its own L2 and
@@ -616,8 +629,8 @@ template <class R>
 __global__ QVNT_FUSED_BOUNDS void k_fused(cplx<R>* __restrict__ psi, FPass pass, const FPhase* __restrict__ phases,
                                                const FOp* __restrict__ ops, const double* __restrict__ coef) {
     extern __shared__ unsigned char smem[];
-    fused_tile<R, true>(psi, pass, phases, ops, coef, xcd_order(blockIdx.x, gridDim.x), reinterpret_cast<cplx<R>*>(smem),
-                        threadIdx.x);
+    fused_tile<R>(psi, pass, phases, ops, coef, xcd_order(blockIdx.x, gridDim.x), gridDim.x,
+                  reinterpret_cast<R*>(smem), threadIdx.x);
 }
 
 // The batched form: the tiles of one pass of many registers in one launch
@@ -640,10 +653,9 @@ __global__ QVNT_FUSED_BOUNDS void k_batch(cplx<R>* __restrict__ arena, const uns
         // the tile's first LDS writes may hit elements other threads still
         // read in the previous tile's last phase
         if (k) __syncthreads();
-        fused_tile<R, false>(arena + it.psi_off, pass, reinterpret_cast<const FPhase*>(prog + it.phase_off),
-                             reinterpret_cast<const FOp*>(prog + it.op_off),
-                             reinterpret_cast<const double*>(prog + it.coef_off), tile, reinterpret_cast<cplx<R>*>(smem),
-                             threadIdx.x);
+        fused_tile<R>(arena + it.psi_off, pass, reinterpret_cast<const FPhase*>(prog + it.phase_off),
+                      reinterpret_cast<const FOp*>(prog + it.op_off), reinterpret_cast<const double*>(prog + it.coef_off), tile,
+                      k ? ~0u : it.tiles, reinterpret_cast<R*>(smem), threadIdx.x);
     }
 }
 
@@ -667,13 +679,13 @@ __device__ __forceinline__ void persist_unit(cplx<R>* __restrict__ arena, const 
     if (tbits >= 6) {
         const uint32_t group = __builtin_amdgcn_readfirstlane(threadIdx.x >> tbits);
         const uint32_t tile = un.tile0 + group;
-        fused_tile<R, false, true>(arena + it.psi_off, pass, ph, ops, coef, tile,
-                                   reinterpret_cast<cplx<R>*>(smem) + ((size_t)group << pass.t), tid, tile < un.tile_end);
+        fused_tile<R, true>(arena + it.psi_off, pass, ph, ops, coef, tile, ~0u,
+                            reinterpret_cast<R*>(smem) + ((size_t)group << pass.t), tid, tile < un.tile_end);
     } else {
         const uint32_t group = threadIdx.x >> tbits;
         const uint32_t tile = un.tile0 + group;
-        fused_tile<R, false, true>(arena + it.psi_off, pass, ph, ops, coef, tile,
-                                   reinterpret_cast<cplx<R>*>(smem) + ((size_t)group << pass.t), tid, tile < un.tile_end);
+        fused_tile<R, true>(arena + it.psi_off, pass, ph, ops, coef, tile, ~0u,
+                            reinterpret_cast<R*>(smem) + ((size_t)group << pass.t), tid, tile < un.tile_end);
     }
 }
 
@@ -706,8 +718,8 @@ constexpr uint32_t kPersistChunk = 4;
 // tile's 16-byte accesses need it (an array at byte 4 made every run 35 %
 // slower).
 //
-// The launch bounds are k_fused's: they leave the register allocation at
-// what the kernel uses, which is what the runtime's occupancy query (and so
+// The launch bounds ask for no minimum of waves: the register allocation
+// stays at what the kernel uses, which is what the runtime's occupancy query (and so
 // the cooperative grid size) counts.
 //
 // A launch that is not cooperative (a graph node whose cooperative
@@ -715,7 +727,7 @@ constexpr uint32_t kPersistChunk = 4;
 // sees that alike, block 0 sets *status to 1, and all return before any
 // barrier or HBM access.
 template <class R>
-__global__ QVNT_FUSED_BOUNDS void k_batch_persist(cplx<R>* __restrict__ arena, const unsigned char* __restrict__ prog,
+__global__ QVNT_PERSIST_BOUNDS void k_batch_persist(cplx<R>* __restrict__ arena, const unsigned char* __restrict__ prog,
                                                   const BItem* __restrict__ items, const PUnit* __restrict__ units,
                                                   const uint32_t* __restrict__ round_begin, uint32_t rounds,
                                                   uint32_t* status) {
@@ -773,11 +785,11 @@ __global__ QVNT_FUSED_BOUNDS void k_batch_persist(cplx<R>* __restrict__ arena, c
 
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-struct Layout {
+struct ProgramLayout {
     size_t ph_off, op_off, cf_off, total;
 };
-Layout layout_of(const Program& prog) {
-    Layout L;
+ProgramLayout program_layout(const Program& prog) {
+    ProgramLayout L;
     L.ph_off = 0;
     L.op_off = align256(L.ph_off + prog.phases.size() * sizeof(FPhase));
     L.cf_off = align256(L.op_off + prog.ops.size() * sizeof(FOp));
@@ -787,12 +799,12 @@ Layout layout_of(const Program& prog) {
 
 }  // namespace
 
-size_t program_bytes(const Program& prog) { return layout_of(prog).total; }
+size_t program_bytes(const Program& prog) { return program_layout(prog).total; }
 
 int batch_persist_grid(qvnt_prec prec, uint32_t tmax, uint32_t* blocks) {
     const size_t amp = prec == QVNT_F64 ? 16 : 8;
     const int threads = 1 << (tmax - kRegBits);
-    const size_t lds = ((size_t)1 << tmax) * amp;
+    const size_t lds = ((size_t)1 << tmax) * amp / 2;
     int per_cu = 0, dev = 0, cus = 0, coop = 0;
     QVNT_HIP(hipGetDevice(&dev));
     QVNT_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
@@ -803,6 +815,10 @@ int batch_persist_grid(qvnt_prec prec, uint32_t tmax, uint32_t* blocks) {
     else
         QVNT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_persist<float>, threads, lds));
     if (per_cu <= 0) return fail(QVNT_E_HIP, "the persistent batched kernel does not fit a compute unit");
+    // three waves per SIMD (QVNT_PERSIST_BOUNDS): more resident blocks only
+    // lengthen the grid barriers
+    const int most = 12 / (threads < 64 ? 1 : threads / 64);
+    if (per_cu > most && most > 0) per_cu = most;
     *blocks = (uint32_t)per_cu * (uint32_t)cus;
     return QVNT_OK;
 }
@@ -812,7 +828,7 @@ int launch_batch_persist(hipStream_t stream, qvnt_prec prec, void* arena, const 
                          uint32_t blocks, uint32_t* status, hipGraph_t* graph) {
     const size_t amp = prec == QVNT_F64 ? 16 : 8;
     const dim3 grid(blocks), block(1u << (tmax - kRegBits));
-    const size_t lds = ((size_t)1 << tmax) * amp;
+    const size_t lds = ((size_t)1 << tmax) * amp / 2;
     const unsigned char* p = static_cast<const unsigned char*>(prog);
     void* args[] = {&arena, &p, &items, &units, &round_begin, &rounds, &status};
     void* fn = prec == QVNT_F64 ? reinterpret_cast<void*>(k_batch_persist<double>)
@@ -842,7 +858,7 @@ int launch_batch(hipStream_t stream, qvnt_prec prec, void* arena, const void* pr
                  uint32_t t, uint32_t blocks) {
     const size_t amp = prec == QVNT_F64 ? 16 : 8;
     const dim3 grid(blocks), block(1u << (t - kRegBits));
-    const size_t lds = ((size_t)1 << t) * amp;
+    const size_t lds = ((size_t)1 << t) * amp / 2;
     const unsigned char* p = static_cast<const unsigned char*>(prog);
     if (prec == QVNT_F64)
         hipLaunchKernelGGL(k_batch<double>, grid, block, lds, stream, static_cast<c64*>(arena), p, items, map);
@@ -853,7 +869,7 @@ int launch_batch(hipStream_t stream, qvnt_prec prec, void* arena, const void* pr
 }
 
 void pack_program(const Program& prog, unsigned char* host) {
-    const Layout L = layout_of(prog);
+    const ProgramLayout L = program_layout(prog);
     std::memset(host, 0, L.total);
     if (!prog.phases.empty()) std::memcpy(host + L.ph_off, prog.phases.data(), prog.phases.size() * sizeof(FPhase));
     if (!prog.ops.empty()) std::memcpy(host + L.op_off, prog.ops.data(), prog.ops.size() * sizeof(FOp));
@@ -861,14 +877,14 @@ void pack_program(const Program& prog, unsigned char* host) {
 }
 
 int launch_program(qvnt_reg* r, const Program& prog, const void* dev) {
-    const Layout L = layout_of(prog);
+    const ProgramLayout L = program_layout(prog);
     const unsigned char* d = static_cast<const unsigned char*>(dev);
     const FPhase* dph = reinterpret_cast<const FPhase*>(d + L.ph_off);
     const FOp* dop = reinterpret_cast<const FOp*>(d + L.op_off);
     const double* dcf = reinterpret_cast<const double*>(d + L.cf_off);
     for (const FPass& fp : prog.passes) {
         const uint64_t tiles = r->len >> fp.t;
-        const size_t lds = ((size_t)1 << fp.t) * r->amp_bytes();
+        const size_t lds = ((size_t)1 << fp.t) * r->amp_bytes() / 2;
         Timed t(r, QVNT_K_FUSED, 2.0 * (double)r->amp_bytes() * (double)r->len);
         if (r->prec == QVNT_F64)
             hipLaunchKernelGGL(k_fused<double>, dim3((unsigned)tiles), dim3(fp.nthreads), lds, r->stream,
