@@ -94,7 +94,7 @@ unsigned single_share(const qvnt_gate& g, unsigned ns, bool fp64) {
 
 }  // namespace
 
-Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run* run) {
+Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, unsigned regs, unsigned max_tile, Run* run) {
     Prim prims[kMaxPrims];
     while (*pos < n && lower(g[*pos], ns, prims) == 0) ++*pos;
     Step step;
@@ -106,25 +106,25 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
         ++*pos;
         return step;
     }
-    const unsigned tmax = ns < max_tile(fp64) ? ns : max_tile(fp64);
-    const unsigned rows = row_bits(fp64) + kRegBits < tmax ? row_bits(fp64) : tmax - kRegBits;
+    const unsigned tmax = ns < max_tile ? ns : max_tile;
+    const unsigned rows = row_bits(fp64) + regs < tmax ? row_bits(fp64) : tmax - regs;
 
     // the longest prefix of the queue that fits: its tile qubits, and its
     // phases' register qubits
     Prim list[kMaxOps];
-    uint64_t regs[kMaxPhases];
+    uint64_t mixed[kMaxPhases];
     unsigned ends[kMaxPhases];
     unsigned count = 0, phases = 1, share = 0;
     uint64_t tile = (1ull << rows) - 1u;
-    regs[0] = 0;
+    mixed[0] = 0;
     size_t i = *pos, last = *pos, gates = 0;
     for (; i < n; ++i) {
         const int k = lower(g[i], ns, prims);
         if (k < 0) break;
         if (k == 0) continue;
         unsigned c2 = count, ph2 = phases;
-        uint64_t t2 = tile, r2 = regs[phases - 1];
-        uint64_t nregs[kMaxPhases];
+        uint64_t t2 = tile, r2 = mixed[phases - 1];
+        uint64_t nmixed[kMaxPhases];
         unsigned nends[kMaxPhases];
         bool ok = true;
         for (int j = 0; j < k && ok; ++j) {
@@ -132,10 +132,10 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
             t2 |= p.mix;
             ok = c2 < kMaxOps && popc(t2) <= tmax;
             if (!ok) break;
-            if (popc(r2 | p.mix) > kRegBits) {
+            if (popc(r2 | p.mix) > regs) {
                 ok = ph2 < kMaxPhases;
                 if (!ok) break;
-                nregs[ph2 - 1] = r2;
+                nmixed[ph2 - 1] = r2;
                 nends[ph2 - 1] = c2;
                 ++ph2;
                 r2 = 0;
@@ -145,10 +145,10 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
         }
         if (!ok) break;
         for (unsigned q = phases; q < ph2; ++q) {
-            regs[q - 1] = nregs[q - 1];
+            mixed[q - 1] = nmixed[q - 1];
             ends[q - 1] = nends[q - 1];
         }
-        regs[ph2 - 1] = r2;
+        mixed[ph2 - 1] = r2;
         count = c2;
         phases = ph2;
         tile = t2;
@@ -171,6 +171,7 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
     for (unsigned q = 0; popc(tile) < tmax; ++q) tile |= 1ull << q;
     std::memset(run, 0, sizeof(Run));
     run->t = tmax;
+    run->regs = regs;
     run->nphases = phases;
     run->nops = count;
     int local[64];
@@ -191,8 +192,8 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
     unsigned c = 0;
     for (unsigned ph = 0; ph < phases; ++ph) {
         // register bits: the phase's own, then the tile's top bits
-        uint32_t rl = local_mask(regs[ph]);
-        for (int b = (int)t - 1; popc(rl) < kRegBits; --b) rl |= 1u << b;
+        uint32_t rl = local_mask(mixed[ph]);
+        for (int b = (int)t - 1; popc(rl) < regs; --b) rl |= 1u << b;
         int reg[kMaxTile];
         unsigned j = 0;
         for (unsigned b = 0; b < t; ++b) {
@@ -212,7 +213,7 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
             const uint32_t lc = local_mask(p.ctrl), lp = local_mask(p.parity);
             const uint32_t rc = reg_mask(lc);
             uint32_t pc = 0;
-            for (uint32_t r = 0; r < kRegs; ++r)
+            for (uint32_t r = 0; r < 1u << regs; ++r)
                 if ((r & rc) == rc) pc |= 1u << r;
             uint32_t variant = reg_mask(local_mask(p.mix));
             if (p.family == F_RZ) variant = reg_mask(lp);
@@ -223,19 +224,21 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, Run
             op.im = p.im;
             run->outer[c].ctrl = p.ctrl & ~tile;
             run->outer[c].parity = p.parity & ~tile;
-            if (run->outer[c].ctrl | run->outer[c].parity) run->outside = 1;
         }
         run->phase[ph].op_end = (uint16_t)c;
     }
     // the tile is read and written in the first and last phase's layout
     // where that keeps the bits of a line among the threads, else with its
     // top bits in the registers
-    const auto edge = [&](const RPhase& ph, uint8_t* to) {
+    const auto edge = [&](const RPhase& ph, uint8_t* to, uint8_t* global) {
         const bool own = ph.rpos[0] >= rows;
-        for (unsigned j = 0; j < kRegBits; ++j) to[j] = own ? ph.rpos[j] : (uint8_t)(t - kRegBits + j);
+        for (unsigned j = 0; j < regs; ++j) {
+            to[j] = own ? ph.rpos[j] : (uint8_t)(t - regs + j);
+            global[j] = run->tpos[to[j]];
+        }
     };
-    edge(run->phase[0], run->in);
-    edge(run->phase[phases - 1], run->out);
+    edge(run->phase[0], run->in, run->gin);
+    edge(run->phase[phases - 1], run->out, run->gout);
     return step;
 }
 

@@ -1,13 +1,16 @@
-// One SingleOp of a run on the 16 amplitudes a thread holds (runs.hpp): the
+// One SingleOp of a run on the 2^B amplitudes a thread holds (runs.hpp): the
 // formulas of device.hpp on the register array, every index known at
 // compile time.
 #pragma once
 
 #include "device.hpp"
 #include "runs.hpp"
+#include "tile.hpp"
 
 namespace qvnt {
 namespace runs {
+
+using tile::put;
 
 QVNT_HD Par par_of(double re, double im, uint32_t a, bool dagger) {
     Par g{};
@@ -19,26 +22,12 @@ QVNT_HD Par par_of(double re, double im, uint32_t a, bool dagger) {
     return g;
 }
 
-// The new value of an amplitude, in its register: kept back on lanes that
-// the gate does not act on (M: there may be some).  The empty asm ends the
-// orbit's update: nothing of the next orbit is computed before.  Without it
-// the scheduler holds the inputs and outputs of all 16 amplitudes at once,
-// in FP64 more than the 128 registers of four waves per SIMD.
-template <bool M, class R>
-QVNT_HD void put(cplx<R>& x, cplx<R> now, bool on) {
-    x.re = !M || on ? now.re : x.re;
-    x.im = !M || on ? now.im : x.im;
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(x.re), "+v"(x.im));
-#endif
-}
-
 // one register bit J, at the register indices of pc (M: not all of them, or
 // not on all lanes)
-template <int K, int J, bool M, class R>
+template <int B, int K, int J, bool M, class R>
 QVNT_HD void one_bit(cplx<R>* v, uint32_t pc, bool on, const Par& g) {
 #pragma unroll
-    for (int i = 0; i < (int)kRegs; ++i) {
+    for (int i = 0; i < 1 << B; ++i) {
         if (i & (1 << J)) continue;
         if (M && !((pc >> i) & 1u)) continue;
         const cplx<R> x0 = v[i], x1 = v[i | (1 << J)];
@@ -46,54 +35,54 @@ QVNT_HD void one_bit(cplx<R>* v, uint32_t pc, bool on, const Par& g) {
         put<M>(v[i | (1 << J)], f_pair<K>(g, 1, x1, x0), on);
     }
 }
-template <int K, bool M, class R>
+template <int B, int K, bool M, class R>
 QVNT_HD void one_bit_sel(cplx<R>* v, uint32_t j, uint32_t pc, bool on, const Par& g) {
     switch (j) {
-    case 0: one_bit<K, 0, M>(v, pc, on, g); break;
-    case 1: one_bit<K, 1, M>(v, pc, on, g); break;
-    case 2: one_bit<K, 2, M>(v, pc, on, g); break;
-    default: one_bit<K, 3, M>(v, pc, on, g); break;
+    case 0: one_bit<B, K, 0, M>(v, pc, on, g); break;
+    case 1: one_bit<B, K, 1, M>(v, pc, on, g); break;
+    case 2: one_bit<B, K, 2, M>(v, pc, on, g); break;
+    default: if constexpr (B > 3) one_bit<B, K, 3, M>(v, pc, on, g); break;
     }
 }
 
-// two register bits, mask B: both parities' pairs (r, r ^ 3), or the odd one only
-template <int K, int B, bool ODD, bool M, class R>
+// two register bits, mask P: both parities' pairs (r, r ^ 3), or the odd one only
+template <int B, int K, int P, bool ODD, bool M, class R>
 QVNT_HD void two_bit(cplx<R>* v, uint32_t pc, bool on, const Par& g) {
-    constexpr int lo = B & -B, hi = B ^ lo;
+    constexpr int lo = P & -P, hi = P ^ lo;
 #pragma unroll
-    for (int i = 0; i < (int)kRegs; ++i) {
-        if (i & B) continue;
+    for (int i = 0; i < 1 << B; ++i) {
+        if (i & P) continue;
         if (M && !((pc >> i) & 1u)) continue;
         if (!ODD) {
-            const cplx<R> x0 = v[i], x3 = v[i | B];
+            const cplx<R> x0 = v[i], x3 = v[i | P];
             put<M>(v[i], f_pair<K>(g, 0, x0, x3), on);
-            put<M>(v[i | B], f_pair<K>(g, 3, x3, x0), on);
+            put<M>(v[i | P], f_pair<K>(g, 3, x3, x0), on);
         }
         const cplx<R> x1 = v[i | lo], x2 = v[i | hi];
         put<M>(v[i | lo], f_pair<K>(g, 1, x1, x2), on);
         put<M>(v[i | hi], f_pair<K>(g, 2, x2, x1), on);
     }
 }
-template <int K, bool ODD, bool M, class R>
+template <int B, int K, bool ODD, bool M, class R>
 QVNT_HD void two_bit_sel(cplx<R>* v, uint32_t b, uint32_t pc, bool on, const Par& g) {
     switch (b) {
-    case 3: two_bit<K, 3, ODD, M>(v, pc, on, g); break;
-    case 5: two_bit<K, 5, ODD, M>(v, pc, on, g); break;
-    case 6: two_bit<K, 6, ODD, M>(v, pc, on, g); break;
-    case 9: two_bit<K, 9, ODD, M>(v, pc, on, g); break;
-    case 10: two_bit<K, 10, ODD, M>(v, pc, on, g); break;
-    default: two_bit<K, 12, ODD, M>(v, pc, on, g); break;
+    case 3: two_bit<B, K, 3, ODD, M>(v, pc, on, g); break;
+    case 5: two_bit<B, K, 5, ODD, M>(v, pc, on, g); break;
+    case 6: two_bit<B, K, 6, ODD, M>(v, pc, on, g); break;
+    case 9: if constexpr (B > 3) two_bit<B, K, 9, ODD, M>(v, pc, on, g); break;
+    case 10: if constexpr (B > 3) two_bit<B, K, 10, ODD, M>(v, pc, on, g); break;
+    default: if constexpr (B > 3) two_bit<B, K, 12, ODD, M>(v, pc, on, g); break;
     }
 }
 
 // h2 (h2.rs:22-38): slot bit 0 is the gate's a, the lower register bit
 // unless REV
-template <int B, bool REV, bool M, class R>
+template <int B, int P, bool REV, bool M, class R>
 QVNT_HD void quad(cplx<R>* v, uint32_t pc, bool on) {
-    constexpr int lo = B & -B, hi = B ^ lo, a = REV ? hi : lo, b = REV ? lo : hi;
+    constexpr int lo = P & -P, hi = P ^ lo, a = REV ? hi : lo, b = REV ? lo : hi;
 #pragma unroll
-    for (int i = 0; i < (int)kRegs; ++i) {
-        if (i & B) continue;
+    for (int i = 0; i < 1 << B; ++i) {
+        if (i & P) continue;
         if (M && !((pc >> i) & 1u)) continue;
         const c64 x[4] = {up(v[i]), up(v[i | a]), up(v[i | b]), up(v[i | a | b])};
         put<M>(v[i], down<R>(f_h2_rel(0, x[0], x[1], x[2], x[3])), on);
@@ -102,51 +91,51 @@ QVNT_HD void quad(cplx<R>* v, uint32_t pc, bool on) {
         put<M>(v[i | a | b], down<R>(f_h2_rel(3, x[3], x[2], x[1], x[0])), on);
     }
 }
-template <bool REV, bool M, class R>
+template <int B, bool REV, bool M, class R>
 QVNT_HD void quad_sel(cplx<R>* v, uint32_t b, uint32_t pc, bool on) {
     switch (b) {
-    case 3: quad<3, REV, M>(v, pc, on); break;
-    case 5: quad<5, REV, M>(v, pc, on); break;
-    case 6: quad<6, REV, M>(v, pc, on); break;
-    case 9: quad<9, REV, M>(v, pc, on); break;
-    case 10: quad<10, REV, M>(v, pc, on); break;
-    default: quad<12, REV, M>(v, pc, on); break;
+    case 3: quad<B, 3, REV, M>(v, pc, on); break;
+    case 5: quad<B, 5, REV, M>(v, pc, on); break;
+    case 6: quad<B, 6, REV, M>(v, pc, on); break;
+    case 9: if constexpr (B > 3) quad<B, 9, REV, M>(v, pc, on); break;
+    case 10: if constexpr (B > 3) quad<B, 10, REV, M>(v, pc, on); break;
+    default: if constexpr (B > 3) quad<B, 12, REV, M>(v, pc, on); break;
     }
 }
 
 // rz / rzz (rz.rs:19-25, rzz.rs:19-25): the phase's imaginary part is im
 // where the act bits have odd parity, -im where even; imx is the value for
-// even parity of the register bits among them, B
-template <int B, bool M, class R>
+// even parity of the register bits among them, P
+template <int B, int P, bool M, class R>
 QVNT_HD void parity_phase(cplx<R>* v, uint32_t pc, bool on, double re, double imx) {
 #pragma unroll
-    for (int i = 0; i < (int)kRegs; ++i) {
+    for (int i = 0; i < 1 << B; ++i) {
         if (M && !((pc >> i) & 1u)) continue;
-        put<M>(v[i], down<R>(cmul(c64{re, (__builtin_popcount(i & B) & 1) ? -imx : imx}, up(v[i]))), on);
+        put<M>(v[i], down<R>(cmul(c64{re, (__builtin_popcount(i & P) & 1) ? -imx : imx}, up(v[i]))), on);
     }
 }
-template <bool M, class R>
+template <int B, bool M, class R>
 QVNT_HD void parity_phase_sel(cplx<R>* v, uint32_t b, uint32_t pc, bool on, double re, double imx) {
     switch (b) {
-    case 0: parity_phase<0, M>(v, pc, on, re, imx); break;
-    case 1: parity_phase<1, M>(v, pc, on, re, imx); break;
-    case 2: parity_phase<2, M>(v, pc, on, re, imx); break;
-    case 3: parity_phase<3, M>(v, pc, on, re, imx); break;
-    case 4: parity_phase<4, M>(v, pc, on, re, imx); break;
-    case 5: parity_phase<5, M>(v, pc, on, re, imx); break;
-    case 6: parity_phase<6, M>(v, pc, on, re, imx); break;
-    case 8: parity_phase<8, M>(v, pc, on, re, imx); break;
-    case 9: parity_phase<9, M>(v, pc, on, re, imx); break;
-    case 10: parity_phase<10, M>(v, pc, on, re, imx); break;
-    default: parity_phase<12, M>(v, pc, on, re, imx); break;
+    case 0: parity_phase<B, 0, M>(v, pc, on, re, imx); break;
+    case 1: parity_phase<B, 1, M>(v, pc, on, re, imx); break;
+    case 2: parity_phase<B, 2, M>(v, pc, on, re, imx); break;
+    case 3: parity_phase<B, 3, M>(v, pc, on, re, imx); break;
+    case 4: parity_phase<B, 4, M>(v, pc, on, re, imx); break;
+    case 5: parity_phase<B, 5, M>(v, pc, on, re, imx); break;
+    case 6: parity_phase<B, 6, M>(v, pc, on, re, imx); break;
+    case 8: if constexpr (B > 3) parity_phase<B, 8, M>(v, pc, on, re, imx); break;
+    case 9: if constexpr (B > 3) parity_phase<B, 9, M>(v, pc, on, re, imx); break;
+    case 10: if constexpr (B > 3) parity_phase<B, 10, M>(v, pc, on, re, imx); break;
+    default: if constexpr (B > 3) parity_phase<B, 12, M>(v, pc, on, re, imx); break;
     }
 }
 
 // the kinds that scale the amplitudes of pc one by one
-template <uint32_t F, class R>
+template <int B, uint32_t F, class R>
 QVNT_HD void phase(cplx<R>* v, uint32_t pc, bool on, double re, double im) {
 #pragma unroll
-    for (int i = 0; i < (int)kRegs; ++i) {
+    for (int i = 0; i < 1 << B; ++i) {
         if (!((pc >> i) & 1u)) continue;
         const c64 p = up(v[i]), e{kFrac1Sqrt2, kFrac1Sqrt2};
         put<true>(v[i], down<R>(F == F_PH ? cmul(c64{re, im}, p) : F == F_T ? cmul(e, p) : F == F_TD ? cmul(e, rotate(p, 3))
@@ -157,34 +146,34 @@ QVNT_HD void phase(cplx<R>* v, uint32_t pc, bool on, double re, double im) {
 // One op on v.  code, pc: uniform; on: whether the lane's bits satisfy the
 // controls (M false: all lanes do, and pc is full); odd: the parity of the
 // act bits outside the registers (per lane).
-template <bool M, class R>
+template <int B, bool M, class R>
 QVNT_HD void apply_op(cplx<R>* v, uint32_t code, uint32_t pc, bool on, bool odd, double re, double im) {
     const uint32_t f = code >> 4, var = code & 15u;
     const Par g1 = par_of(re, im, 1u, false), g2 = par_of(re, im, 3u, false), g2d = par_of(re, im, 3u, true);
     switch (f) {
-    case F_PH: phase<F_PH>(v, pc, on, re, im); break;
-    case F_I1: phase<F_I1>(v, pc, on, re, im); break;
-    case F_I2: phase<F_I2>(v, pc, on, re, im); break;
-    case F_I3: phase<F_I3>(v, pc, on, re, im); break;
-    case F_T: phase<F_T>(v, pc, on, re, im); break;
-    case F_TD: phase<F_TD>(v, pc, on, re, im); break;
-    case F_RZ: parity_phase_sel<M>(v, var, pc, on, re, odd ? im : -im); break;
-    case F_X: one_bit_sel<QVNT_X, M>(v, var, pc, on, g1); break;
-    case F_Y: one_bit_sel<QVNT_Y, M>(v, var, pc, on, g1); break;
-    case F_RX: one_bit_sel<QVNT_RX, M>(v, var, pc, on, g1); break;
-    case F_RY: one_bit_sel<QVNT_RY, M>(v, var, pc, on, g1); break;
-    case F_H1: one_bit_sel<QVNT_H1, M>(v, var, pc, on, g1); break;
-    case F_RXX: two_bit_sel<QVNT_RXX, false, M>(v, var, pc, on, g2); break;
-    case F_RYY: two_bit_sel<QVNT_RYY, false, M>(v, var, pc, on, g2); break;
-    case F_SWAP: two_bit_sel<QVNT_SWAP, true, M>(v, var, pc, on, g2); break;
-    case F_ISWAP: two_bit_sel<QVNT_ISWAP, true, M>(v, var, pc, on, g2); break;
-    case F_ISWAPD: two_bit_sel<QVNT_ISWAP, true, M>(v, var, pc, on, g2d); break;
-    case F_SQSW: two_bit_sel<QVNT_SQRT_SWAP, true, M>(v, var, pc, on, g2); break;
-    case F_SQSWD: two_bit_sel<QVNT_SQRT_SWAP, true, M>(v, var, pc, on, g2d); break;
-    case F_SQIS: two_bit_sel<QVNT_SQRT_ISWAP, true, M>(v, var, pc, on, g2); break;
-    case F_SQISD: two_bit_sel<QVNT_SQRT_ISWAP, true, M>(v, var, pc, on, g2d); break;
-    case F_H2: quad_sel<false, M>(v, var, pc, on); break;
-    default: quad_sel<true, M>(v, var, pc, on); break;
+    case F_PH: phase<B, F_PH>(v, pc, on, re, im); break;
+    case F_I1: phase<B, F_I1>(v, pc, on, re, im); break;
+    case F_I2: phase<B, F_I2>(v, pc, on, re, im); break;
+    case F_I3: phase<B, F_I3>(v, pc, on, re, im); break;
+    case F_T: phase<B, F_T>(v, pc, on, re, im); break;
+    case F_TD: phase<B, F_TD>(v, pc, on, re, im); break;
+    case F_RZ: parity_phase_sel<B, M>(v, var, pc, on, re, odd ? im : -im); break;
+    case F_X: one_bit_sel<B, QVNT_X, M>(v, var, pc, on, g1); break;
+    case F_Y: one_bit_sel<B, QVNT_Y, M>(v, var, pc, on, g1); break;
+    case F_RX: one_bit_sel<B, QVNT_RX, M>(v, var, pc, on, g1); break;
+    case F_RY: one_bit_sel<B, QVNT_RY, M>(v, var, pc, on, g1); break;
+    case F_H1: one_bit_sel<B, QVNT_H1, M>(v, var, pc, on, g1); break;
+    case F_RXX: two_bit_sel<B, QVNT_RXX, false, M>(v, var, pc, on, g2); break;
+    case F_RYY: two_bit_sel<B, QVNT_RYY, false, M>(v, var, pc, on, g2); break;
+    case F_SWAP: two_bit_sel<B, QVNT_SWAP, true, M>(v, var, pc, on, g2); break;
+    case F_ISWAP: two_bit_sel<B, QVNT_ISWAP, true, M>(v, var, pc, on, g2); break;
+    case F_ISWAPD: two_bit_sel<B, QVNT_ISWAP, true, M>(v, var, pc, on, g2d); break;
+    case F_SQSW: two_bit_sel<B, QVNT_SQRT_SWAP, true, M>(v, var, pc, on, g2); break;
+    case F_SQSWD: two_bit_sel<B, QVNT_SQRT_SWAP, true, M>(v, var, pc, on, g2d); break;
+    case F_SQIS: two_bit_sel<B, QVNT_SQRT_ISWAP, true, M>(v, var, pc, on, g2); break;
+    case F_SQISD: two_bit_sel<B, QVNT_SQRT_ISWAP, true, M>(v, var, pc, on, g2d); break;
+    case F_H2: quad_sel<B, false, M>(v, var, pc, on); break;
+    default: quad_sel<B, true, M>(v, var, pc, on); break;
     }
 }
 

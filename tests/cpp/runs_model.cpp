@@ -33,28 +33,31 @@ bool is_diagonal_kind(uint32_t) { return false; }
 }
 
 static uint32_t swz(uint32_t e) { return e ^ (e >> 4); }
+template <int B>
 static uint32_t spread(uint32_t x, const uint8_t* p) {
-    for (unsigned j = 0; j < kRegBits; ++j) {
+    for (unsigned j = 0; j < B; ++j) {
         if (j) CHECK(p[j] > p[j - 1]);
         const uint32_t lo = x & ((1u << p[j]) - 1u);
         x = ((x ^ lo) << 1) | lo;
     }
     return x;
 }
+template <int B>
 static uint32_t element(uint32_t tid, int i, const uint8_t* p) {
-    uint32_t e = spread(tid, p);
-    for (unsigned j = 0; j < kRegBits; ++j)
+    uint32_t e = spread<B>(tid, p);
+    for (unsigned j = 0; j < B; ++j)
         if (i >> j & 1) e |= 1u << p[j];
     return e;
 }
 
-static int seen[F_COUNT][2];
+static int seen[F_COUNT][2][2];
 
-template <class R>
+template <int B, class R>
 static void run_step(std::vector<cplx<R>>& psi, unsigned ns, const Run& run) {
-    const unsigned t = run.t, nth = 1u << (t - kRegBits);
-    CHECK(t >= kRegBits && t <= kMaxTile && t <= ns && run.nphases >= 1 && run.nphases <= kMaxPhases && run.nops <= kMaxOps);
+    const unsigned t = run.t, nth = 1u << (t - B);
+    CHECK(run.regs == B && t >= B && t <= kMaxTile && t <= ns && run.nphases >= 1 && run.nphases <= kMaxPhases && run.nops <= kMaxOps);
     for (unsigned k = 0; k + 1 < t; ++k) CHECK(run.tpos[k] < run.tpos[k + 1] && run.tpos[k + 1] < ns);
+    for (int j = 0; j < B; ++j) CHECK(run.gin[j] == run.tpos[run.in[j]] && run.gout[j] == run.tpos[run.out[j]]);
     std::vector<char> hit(1u << t, 0);
     for (uint32_t e = 0; e < 1u << t; ++e) {
         CHECK(swz(e) < 1u << t && !hit[swz(e)]);
@@ -73,15 +76,15 @@ static void run_step(std::vector<cplx<R>>& psi, unsigned ns, const Run& run) {
         };
         std::vector<cplx<R>> local(1u << t);
         for (uint32_t tid = 0; tid < nth; ++tid)
-            for (int i = 0; i < (int)kRegs; ++i) local[element(tid, i, run.in)] = psi[global(element(tid, i, run.in))];
+            for (int i = 0; i < 1 << B; ++i) local[element<B>(tid, i, run.in)] = psi[global(element<B>(tid, i, run.in))];
         uint32_t o = 0;
         for (uint32_t ph = 0; ph < run.nphases; ++ph) {
             const RPhase& p = run.phase[ph];
-            CHECK(p.op_end >= o && p.op_end <= run.nops && p.rpos[kRegBits - 1] < t);
+            CHECK(p.op_end >= o && p.op_end <= run.nops && p.rpos[B - 1] < t);
             for (uint32_t tid = 0; tid < nth; ++tid) {
-                cplx<R> v[kRegs];
-                const uint32_t tb = spread(tid, p.rpos);
-                for (int i = 0; i < (int)kRegs; ++i) v[i] = local[element(tid, i, p.rpos)];
+                cplx<R> v[1 << B];
+                const uint32_t tb = spread<B>(tid, p.rpos);
+                for (int i = 0; i < 1 << B; ++i) v[i] = local[element<B>(tid, i, p.rpos)];
                 for (uint32_t k = o; k < p.op_end; ++k) {
                     const ROp& op = run.op[k];
                     const ROut& q = run.outer[k];
@@ -91,18 +94,18 @@ static void run_step(std::vector<cplx<R>>& psi, unsigned ns, const Run& run) {
                     const bool odd = ((dpopc(tb & (op.lbits >> 16)) + dpopc(tile & q.parity)) & 1u) != 0;
                     if (!live) continue;
                     // the kernel's two forms: whole waves, and lanes selected
-                    const bool whole = on && pc == 0xFFFFu && lc == 0;
-                    seen[code >> 4][whole ? 0 : 1] = 1;
-                    if (whole) apply_op<false>(v, code, pc, true, odd, op.re, op.im);
-                    else apply_op<true>(v, code, pc, on, odd, op.re, op.im);
+                    const bool whole = on && pc == (1u << (1 << B)) - 1u && lc == 0;
+                    seen[code >> 4][B - 3][whole ? 0 : 1] = 1;
+                    if (whole) apply_op<B, false>(v, code, pc, true, odd, op.re, op.im);
+                    else apply_op<B, true>(v, code, pc, on, odd, op.re, op.im);
                 }
-                for (int i = 0; i < (int)kRegs; ++i) local[element(tid, i, p.rpos)] = v[i];
+                for (int i = 0; i < 1 << B; ++i) local[element<B>(tid, i, p.rpos)] = v[i];
             }
             o = p.op_end;
         }
         CHECK(o == run.nops);
         for (uint32_t tid = 0; tid < nth; ++tid)
-            for (int i = 0; i < (int)kRegs; ++i) psi[global(element(tid, i, run.out))] = local[element(tid, i, run.out)];
+            for (int i = 0; i < 1 << B; ++i) psi[global(element<B>(tid, i, run.out))] = local[element<B>(tid, i, run.out)];
     }
 }
 
@@ -176,7 +179,7 @@ static std::vector<qvnt_gate> circuit(std::mt19937_64& g, unsigned n, int count,
 }
 
 template <class R>
-static void check(std::mt19937_64& g, unsigned n, int count, bool local, size_t* runs, size_t* singles, size_t* fused) {
+static void check(std::mt19937_64& g, unsigned n, int count, bool local, unsigned regs, size_t* runs, size_t* singles, size_t* fused) {
     const std::vector<qvnt_gate> q = circuit(g, n, count, local);
     const uint64_t len = 1ull << n;
     std::vector<cplx<R>> psi(len);
@@ -199,7 +202,7 @@ static void check(std::mt19937_64& g, unsigned n, int count, bool local, size_t*
     Run run;
     size_t done = 0;
     for (size_t pos = 0;;) {
-        const Step s = next(q.data(), q.size(), &pos, n, sizeof(R) == 8, &run);
+        const Step s = next(q.data(), q.size(), &pos, n, sizeof(R) == 8, regs, regs == 3 ? max_tile(n, sizeof(R) == 8) : max_tile(64, sizeof(R) == 8), &run);
         if (s.kind == Kind::Done) break;
         CHECK(s.from >= done && s.count >= 1 && pos >= s.from + s.count);
         // (gates left out are the identity: the oracle applies them all the same)
@@ -209,7 +212,8 @@ static void check(std::mt19937_64& g, unsigned n, int count, bool local, size_t*
             ++*singles;
             continue;
         }
-        run_step(psi, n, run);
+        if (regs == 3) run_step<3>(psi, n, run);
+        else run_step<4>(psi, n, run);
         ++*runs;
         *fused += s.count;
         for (uint64_t i = 0; i < len; ++i) {
@@ -231,15 +235,18 @@ int main() {
     size_t runs = 0, singles = 0, fused = 0;
     for (unsigned n = 3; n <= 15; ++n)
         for (int k = 0; k < (n < 13 ? 12 : 5); ++k) {
-            check<double>(g, n, 120, k & 1, &runs, &singles, &fused);
-            check<float>(g, n, 120, k & 1, &runs, &singles, &fused);
+            for (unsigned regs = 3; regs <= 4; ++regs) {
+                check<double>(g, n, 120, k & 1, regs, &runs, &singles, &fused);
+                check<float>(g, n, 120, k & 1, regs, &runs, &singles, &fused);
+            }
         }
     for (int f = 0; f < F_COUNT; ++f) {
         const bool whole_possible = f > F_TD;
-        if (!seen[f][1] || (whole_possible && !seen[f][0])) {
-            std::fprintf(stderr, "family %d not run in every form\n", f);
-            return 1;
-        }
+        for (const auto& form : seen[f])
+            if (!form[1] || (whole_possible && !form[0])) {
+                std::fprintf(stderr, "family %d not run in every form\n", f);
+                return 1;
+            }
     }
     std::printf("%zu runs of %zu SingleOps, %zu singles: equal to the oracle\n", runs, fused, singles);
     return 0;
