@@ -9,8 +9,8 @@
 //   node(l,j) = node(l-1,2j) + node(l-1,2j+1)        (pairwise tree),
 //   draw: x = u * node(top,0); from the root, with children (L, R), go left
 //   iff x < L or R == 0, else x -= L and go right; the leaf reached is r.
-// Tree levels from 2^11 leaves upwards are stored (O(2^n / 2^11) doubles);
-// a draw recomputes the 2^11-leaf subtree it lands in.  FP32 registers are
+// Every eleventh level is stored (O(2^n / 2^11) doubles); a draw makes the
+// levels between again on its way down.  FP32 registers are
 // reduced, searched and rescaled in FP64 as well.
 #pragma clang fp contract(off)
 
@@ -29,7 +29,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr unsigned kLeafLog = 11;          // leaves per stored bottom node
-constexpr unsigned kLeaf = 1u << kLeafLog;
 
 template <class R>
 __device__ __forceinline__ double weight(cplx<R> p) {
@@ -37,129 +36,223 @@ __device__ __forceinline__ double weight(cplx<R> p) {
     return re * re + im * im;
 }
 
-// node(11, blockIdx.x): each wave reduces 512 consecutive leaves, 64 per
-// load; lanes pair up with xor-shuffles (adjacent pairs first), then the 8
-// chunk sums and the 4 wave sums pair up in the same adjacent order.
 // A dispatch carries its size in work-items as a 32-bit number: grids are
 // capped at kMaxGrid blocks and kernels stride over their work.
 constexpr uint64_t kMaxGrid = 1u << 20;
+constexpr unsigned kWave = 64;
+constexpr unsigned kBlockWaves = kBlock / kWave;
+constexpr uint64_t kSpreadNodes = 1024;  // 18 qubits: k_leaf 5.2 us in blocks of four waves, 4.5 in blocks of one
 
+// Values of the tree's next lower stored level, or the leaves.
+struct Nodes {
+    const double* p;
+    __device__ __forceinline__ double operator()(uint64_t k) const { return p[k]; }
+};
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_leaf(const cplx<R>* __restrict__ psi, uint64_t nleaves, double* __restrict__ out) {
-  for (uint64_t blk = blockIdx.x; blk < nleaves; blk += gridDim.x) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t base = blk * kLeaf + (uint64_t)wave * 512u;
-    double s[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s[j] = weight(psi[base + (uint64_t)j * 64u + (uint64_t)lane]);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s[j] = s[j] + __shfl_xor(s[j], o);
-    const double w = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
-    __shared__ double sh[4];
-    if (lane == 0) sh[wave] = w;
-    __syncthreads();
-    if (threadIdx.x == 0) out[blk] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-    __syncthreads();
-  }
+struct Leaves {
+    const cplx<R>* p;
+    __device__ __forceinline__ double operator()(uint64_t k) const { return weight(p[k]); }
+};
+
+// The value of lane ^ M.  Within a row of 16 lanes a DPP move where one does
+// it, else an LDS swizzle; every lane of the wave is active.
+template <int M>
+__device__ __forceinline__ int xor_lane(int v) {
+    if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);         // quad_perm 1 0 3 2
+    else if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);    // quad_perm 2 3 0 1
+    else if constexpr (M == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);   // row_ror 8
+    else if constexpr (M < 32) return __builtin_amdgcn_ds_swizzle(v, (M << 10) | 0x1F);
+    else return __shfl_xor(v, M);
+}
+template <int M>
+__device__ __forceinline__ double xor_lane(double v) {
+    return __hiloint2double(xor_lane<M>(__double2hiint(v)), xor_lane<M>(__double2loint(v)));
 }
 
-// Pairwise levels of `span` (<= 2048, a power of two) values held in LDS:
-// lv + off(k) with off(k) = 2*span - (2*span >> k).
-__device__ void lds_levels(double* lv, unsigned span) {
-    unsigned in_off = 0, m = span;
-    while (m > 1) {
-        const unsigned h = m >> 1, out_off = in_off + m;
-        for (unsigned t = threadIdx.x; t < h; t += kBlock) lv[out_off + t] = lv[in_off + 2 * t] + lv[in_off + 2 * t + 1];
-        __syncthreads();
-        in_off = out_off;
-        m = h;
+// Pairwise tree of 64 consecutive values per register, 2^LC registers: at
+// step S lanes whose bit S is 0 go on with the even registers and the others
+// with the odd ones, so each step halves the registers and takes one
+// exchange for two sums.  At the end lane l holds one value, the sum of 2^LC
+// consecutive values: group l >> LC of chunk l & (2^LC - 1).  (All sums of
+// all lanes, six exchanges a register, took k_leaf 4.2 ms in FP32 at 31
+// qubits, 16 GiB: bound by LDS, not by HBM.)
+template <int LC, int S = 0>
+__device__ __forceinline__ void fold(double* a) {
+    if constexpr (S < LC) {
+        const bool odd = (threadIdx.x >> S) & 1u;
+#pragma unroll
+        for (int k = 0; k < 1 << (LC - S - 1); ++k) {
+            const double keep = odd ? a[2 * k + 1] : a[2 * k], give = odd ? a[2 * k] : a[2 * k + 1];
+            a[k] = keep + xor_lane<1 << S>(give);
+        }
+        fold<LC, S + 1>(a);
     }
 }
 
-// Whole tree of a buffer of <= 2048 leaves: writes node(top, 0).
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_small(const cplx<R>* __restrict__ psi, unsigned count, double* __restrict__ out) {
-    __shared__ double lv[2 * kLeaf];
-    for (unsigned t = threadIdx.x; t < count; t += kBlock) lv[t] = weight(psi[t]);
-    __syncthreads();
-    lds_levels(lv, count);
-    if (threadIdx.x == 0) out[0] = lv[2 * count - 2];
+// The rest of the tree: s[d], d = 0 .. 6: this lane's node d levels above
+// fold's (lane bit (LC + d) % 6 pairs level d).
+template <int LC, int D = 0>
+__device__ __forceinline__ void rise(double* s) {
+    if constexpr (D < 6) {
+        s[D + 1] = s[D] + xor_lane<1 << ((LC + D) % 6)>(s[D]);
+        rise<LC, D + 1>(s);
+    }
+}
+// 2^(6 + LC) values (LC 0: 2^lg of them, lg <= 6)
+template <int LC, class F>
+__device__ __forceinline__ void levels(const F& node, uint64_t base, uint32_t lg, double* s) {
+    const uint32_t lane = threadIdx.x & (kWave - 1u);
+    double a[1 << LC];
+#pragma unroll
+    for (int c = 0; c < 1 << LC; ++c) a[c] = LC > 0 || lane < (1u << lg) ? node(base + (uint64_t)c * kWave + lane) : 0.0;
+    fold<LC>(a);
+    s[0] = a[0];
+    rise<LC>(s);
 }
 
-struct LevelPtrs {
-    double* p[kLeafLog + 1];
-};
+// One wave per node of the lowest stored level: 2^11 leaves, all in flight
+// at once, and no barrier.  Bound by HBM: 16 GiB in 2.8 ms, 6.1 TB/s, in FP64
+// and FP32.
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_leaf(const cplx<R>* __restrict__ psi, uint64_t nleaves, double* __restrict__ out) {
+    const uint32_t lane = threadIdx.x & (kWave - 1u);
+    const uint32_t waves = blockDim.x / kWave;
+    for (uint64_t node = (uint64_t)blockIdx.x * waves + threadIdx.x / kWave; node < nleaves; node += (uint64_t)gridDim.x * waves) {
+        double s[7];
+        if constexpr (sizeof(R) == 8) {
+            levels<5>(Leaves<R>{psi}, node << kLeafLog, kLeafLog, s);
+        } else {
+            // two leaves a load
+            const float4* p = reinterpret_cast<const float4*>(psi + (node << kLeafLog)) + lane;
+            double a[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                const float4 q = p[c * (int)kWave];
+                a[c] = weight(c32{q.x, q.y}) + weight(c32{q.z, q.w});
+            }
+            fold<4>(a);
+            s[0] = a[0];
+            rise<4>(s);
+        }
+        if (lane == 0) out[node] = s[6];
+    }
+}
 
-// Levels L+1 .. L+log2(span) above a stored level L of n_in nodes; every
-// block owns `span` consecutive nodes.
-__global__ __launch_bounds__(kBlock) void k_upper(const double* __restrict__ in, unsigned span, LevelPtrs out) {
-    __shared__ double lv[2 * kLeaf];
-    const uint64_t base = (uint64_t)blockIdx.x * span;
-    for (unsigned t = threadIdx.x; t < span; t += kBlock) lv[t] = in[base + t];
-    __syncthreads();
-    lds_levels(lv, span);
-    unsigned off = span, m = span >> 1;
-    for (unsigned k = 1; m >= 1; ++k, off += m, m >>= 1)
-        for (unsigned t = threadIdx.x; t < m; t += kBlock) out.p[k][(uint64_t)blockIdx.x * m + t] = lv[off + t];
+// A stored level from the one 2^11 below it, one wave per node.
+__global__ __launch_bounds__(kBlock) void k_upper(const double* __restrict__ in, uint64_t n, double* __restrict__ out) {
+    const uint64_t node = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    if (node >= n) return;  // uniform over the wave
+    double s[7];
+    levels<5>(Nodes{in}, node << kLeafLog, kLeafLog, s);
+    if ((threadIdx.x & (kWave - 1u)) == 0) out[node] = s[6];
 }
 
 struct TreeInfo {
     uint32_t top;      // log2(count)
     uint32_t lb;       // lowest stored level, min(top, 11)
-    uint64_t off[64];  // offset of stored level l (lb <= l <= top) in the tree array
+    uint64_t off[64];  // offset of level l in the tree array; levels 11, 22, 33 below the top are stored
+};
+// The highest stored level below the top (0: the leaves).
+__host__ __device__ inline uint32_t top_stage(uint32_t top) { return top ? (top - 1u) / kLeafLog * kLeafLog : 0u; }
+
+__device__ __forceinline__ double lane_value(double v, uint32_t lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane), __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// A draw's position: x, what is left of u * total in the node reached.
+struct Draw {
+    double u, x, total;
+    bool first;
 };
 
-// One draw per block: descend the stored levels, then the recomputed
-// 2^lb-leaf subtree of the block reached.  Draw k is u[k], or u0 when u is
-// null (one draw, passed by value: no copy to the device before the launch).
+// Descends the tree over 2^lg values from node(base) (LC 0: lg <= 6, else lg
+// = 6 + LC): the offset of the value reached.  Wave-uniform.
+template <int LC, class F>
+__device__ __forceinline__ uint32_t descend(const F& node, uint64_t base, uint32_t lg, Draw& d) {
+    double s[7];
+    levels<LC>(node, base, lg, s);
+    const uint32_t n = LC ? 6u : lg;
+    if (d.first) {
+        double root = s[6];
+        if (LC == 0) {
+#pragma unroll
+            for (int l = 0; l < 6; ++l) root = n == (uint32_t)l ? s[l] : root;
+        }
+        d.total = lane_value(root, 0);
+        d.x = d.u * d.total;
+        d.first = false;
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int l = 5; l >= 0; --l) {
+        if ((uint32_t)l >= n) continue;  // uniform
+        // the lane that holds node q of level l
+        const auto at = [&](uint32_t q) {
+            const uint32_t i = q << l;
+            return (uint32_t)__builtin_amdgcn_readfirstlane(((i >> (6 - LC)) | (i << LC)) & (kWave - 1u));
+        };
+        const double L = lane_value(s[l], at(2 * m)), R = lane_value(s[l], at(2 * m + 1));
+        const bool left = d.x < L || R == 0.0;
+        d.x = left ? d.x : d.x - L;
+        m = 2 * m + (left ? 0u : 1u);
+    }
+    if constexpr (LC > 0) {
+        const uint32_t first = m << LC;
+        return first + descend<0>(node, base + first, LC, d);
+    } else {
+        return m;
+    }
+}
+template <class F>
+__device__ __forceinline__ uint32_t descend_any(const F& node, uint64_t base, uint32_t lg, Draw& d) {
+    switch (lg) {  // uniform
+    case 7: return descend<1>(node, base, lg, d);
+    case 8: return descend<2>(node, base, lg, d);
+    case 9: return descend<3>(node, base, lg, d);
+    case 10: return descend<4>(node, base, lg, d);
+    case 11: return descend<5>(node, base, lg, d);
+    default: return descend<0>(node, base, lg, d);
+    }
+}
+
+// One draw per wave: down the stored levels, 2^11 nodes at a time, then the
+// leaves of the node reached.  The sums of both are made again in the wave's
+// registers; no barrier, and no chain of loads from one level to the next.
+// Draw k is u[k], or u0 when u is null (one draw, passed by value: no copy to
+// the device before the launch).  1024 draws, FP64: 18 qubits 9.1 us with a block
+// per draw and its levels in LDS, 6.0 now; 20 qubits 13.0 and 11.0; 30 qubits
+// 20 and 17.
 template <class R>
 __global__ __launch_bounds__(kBlock) void k_sample(const cplx<R>* __restrict__ psi, const double* __restrict__ tree,
-                                                   TreeInfo info, const double* __restrict__ u, double u0,
+                                                   TreeInfo info, const double* __restrict__ u, double u0, uint32_t shots,
                                                    uint64_t* __restrict__ out, double* __restrict__ total) {
-    __shared__ double lv[2 * kLeaf];
-    __shared__ uint64_t sj;
-    __shared__ double sx;
-    if (threadIdx.x == 0) {
-        const double T = tree[info.off[info.top]];
-        double x = (u ? u[blockIdx.x] : u0) * T;
-        uint64_t j = 0;
-        for (uint32_t l = info.top; l > info.lb; --l) {
-            const double L = tree[info.off[l - 1] + 2 * j], Rr = tree[info.off[l - 1] + 2 * j + 1];
-            if (x < L || Rr == 0.0) {
-                j = 2 * j;
-            } else {
-                x = x - L;
-                j = 2 * j + 1;
-            }
-        }
-        sj = j;
-        sx = x;
-        if (blockIdx.x == 0) total[0] = T;
+    const uint32_t shot = __builtin_amdgcn_readfirstlane(blockIdx.x * kBlockWaves + threadIdx.x / kWave);
+    if (shot >= shots) return;
+    Draw d{u ? u[shot] : u0, 0.0, 0.0, true};
+    uint64_t j = 0;
+    uint32_t l = info.top;
+    for (uint32_t to = top_stage(info.top); to >= kLeafLog; to -= kLeafLog) {
+        j <<= l - to;
+        j += descend_any(Nodes{tree + info.off[to]}, j, l - to, d);
+        l = to;
     }
-    __syncthreads();
-    const unsigned span = 1u << info.lb;
-    const uint64_t base = sj << info.lb;
-    for (unsigned t = threadIdx.x; t < span; t += kBlock) lv[t] = weight(psi[base + t]);
-    __syncthreads();
-    lds_levels(lv, span);
-    if (threadIdx.x == 0) {
-        double x = sx;
-        uint64_t k = 0;
-        // level l of the block subtree lives at off(l) = 2*span - (2*span >> l)
-        for (uint32_t l = info.lb; l > 0; --l) {
-            const unsigned off = 2 * span - ((2 * span) >> (l - 1));
-            const double L = lv[off + 2 * k], Rr = lv[off + 2 * k + 1];
-            if (x < L || Rr == 0.0) {
-                k = 2 * k;
-            } else {
-                x = x - L;
-                k = 2 * k + 1;
-            }
-        }
-        out[blockIdx.x] = base + k;
+    j <<= l;
+    j += descend_any(Leaves<R>{psi}, j, l, d);
+    if ((threadIdx.x & (kWave - 1u)) == 0) {
+        out[shot] = j;
+        if (shot == 0) total[0] = d.total;
     }
+}
+
+// The root: the sum over the highest stored level, or the leaves.
+template <class R>
+__global__ __launch_bounds__(kWave) void k_total(const cplx<R>* __restrict__ psi, const double* __restrict__ tree, TreeInfo info,
+                                                 double* __restrict__ total) {
+    Draw d{0.0, 0.0, 0.0, true};
+    const uint32_t from = top_stage(info.top);
+    if (from) (void)descend_any(Nodes{tree + info.off[from]}, 0, info.top - from, d);
+    else (void)descend_any(Leaves<R>{psi}, 0, info.top, d);
+    if (threadIdx.x == 0) total[0] = d.total;
 }
 
 // collapse_mask (quant.rs:468-486): zero every amplitude with
@@ -302,33 +395,26 @@ int ensure_workspace(qvnt_reg* r, size_t tree_doubles, size_t shots) {
     return QVNT_OK;
 }
 
-// The tree levels of the first `count` weights into `tree` (laid out by
+// The stored levels of the first `count` weights into `tree` (laid out by
 // tree_info(count)); timed: bracket the launches with the register's timing
 // events (the allocation-free path passes false: it creates no events).
 template <class R>
 int build_levels(qvnt_reg* r, double* tree, uint64_t count, const TreeInfo& info, bool timed) {
-    const cplx<R>* psi = static_cast<const cplx<R>*>(r->psi);
-    qvnt_reg* tr = timed ? r : nullptr;
-    Timed t(tr, QVNT_K_REDUCE, (double)r->amp_bytes() * (double)count);
-    if (info.top < kLeafLog) {
-        hipLaunchKernelGGL(k_small<R>, dim3(1), dim3(kBlock), 0, r->stream, psi, (unsigned)count, tree + info.off[info.top]);
-        QVNT_HIP(hipGetLastError());
-        return QVNT_OK;
-    }
-    const uint64_t nleaves = count >> kLeafLog;
-    hipLaunchKernelGGL(k_leaf<R>, dim3((unsigned)(nleaves < kMaxGrid ? nleaves : kMaxGrid)), dim3(kBlock), 0, r->stream, psi,
-                       nleaves, tree + info.off[kLeafLog]);
+    if (info.top <= kLeafLog) return QVNT_OK;  // the leaves are the level below the top
+    // (few nodes: a wave a block, so that they spread over the CUs)
+    const auto threads = [](uint64_t nodes) { return nodes <= kSpreadNodes ? kWave : (unsigned)kBlock; };
+    const auto grid = [&](uint64_t nodes) {
+        const uint64_t waves = threads(nodes) / kWave, blocks = (nodes + waves - 1) / waves;
+        return dim3((unsigned)(blocks < kMaxGrid ? blocks : kMaxGrid));
+    };
+    Timed t(timed ? r : nullptr, QVNT_K_REDUCE, (double)r->amp_bytes() * (double)count);
+    hipLaunchKernelGGL(k_leaf<R>, grid(count >> kLeafLog), dim3(threads(count >> kLeafLog)), 0, r->stream, static_cast<const cplx<R>*>(r->psi),
+                       count >> kLeafLog, tree + info.off[kLeafLog]);
     QVNT_HIP(hipGetLastError());
-    for (uint32_t L = kLeafLog; L < info.top;) {
-        const uint32_t steps = (info.top - L) < kLeafLog ? (info.top - L) : kLeafLog;
-        const unsigned span = 1u << steps;
-        const uint64_t n_in = count >> L;
-        LevelPtrs lp{};
-        for (uint32_t k = 1; k <= steps; ++k) lp.p[k] = tree + info.off[L + k];
-        hipLaunchKernelGGL(k_upper, dim3((unsigned)(n_in / span)), dim3(kBlock), 0, r->stream,
-                           (const double*)(tree + info.off[L]), span, lp);
+    for (uint32_t l = 2 * kLeafLog; l < info.top; l += kLeafLog) {
+        hipLaunchKernelGGL(k_upper, grid(count >> l), dim3(threads(count >> l)), 0, r->stream, (const double*)(tree + info.off[l - kLeafLog]),
+                           count >> l, tree + info.off[l]);
         QVNT_HIP(hipGetLastError());
-        L += steps;
     }
     return QVNT_OK;
 }
@@ -342,19 +428,22 @@ int sample_into(qvnt_reg* r, double* tree, uint64_t count, const double* u_dev, 
     int rc = r->prec == QVNT_F64 ? build_levels<double>(r, tree, count, info, timed)
                                  : build_levels<float>(r, tree, count, info, timed);
     if (rc) return rc;
+    const dim3 grid((unsigned)((shots + kBlockWaves - 1) / kBlockWaves));
     Timed t(timed ? r : nullptr, QVNT_K_OTHER, 0.0);
     if (r->prec == QVNT_F64)
-        hipLaunchKernelGGL(k_sample<double>, dim3((unsigned)shots), dim3(kBlock), 0, r->stream,
-                           static_cast<const c64*>(r->psi), (const double*)tree, info, u_dev, u0, out_dev, total_dev);
+        hipLaunchKernelGGL(k_sample<double>, grid, dim3(kBlock), 0, r->stream, static_cast<const c64*>(r->psi), (const double*)tree,
+                           info, u_dev, u0, (uint32_t)shots, out_dev, total_dev);
     else
-        hipLaunchKernelGGL(k_sample<float>, dim3((unsigned)shots), dim3(kBlock), 0, r->stream,
-                           static_cast<const c32*>(r->psi), (const double*)tree, info, u_dev, u0, out_dev, total_dev);
+        hipLaunchKernelGGL(k_sample<float>, grid, dim3(kBlock), 0, r->stream, static_cast<const c32*>(r->psi), (const double*)tree,
+                           info, u_dev, u0, (uint32_t)shots, out_dev, total_dev);
     QVNT_HIP(hipGetLastError());
     return QVNT_OK;
 }
 
 }  // namespace
 
+// The total goes straight to pinned host memory where a block is at hand
+// (HostBlock), else through the tree array and a copy.
 int tree_build(qvnt_reg* r, uint64_t count, double* total_out) {
     const TreeInfo info = tree_info(count);
     int rc = ensure_workspace(r, (size_t)(info.off[info.top] + 1), 1);
@@ -362,10 +451,23 @@ int tree_build(qvnt_reg* r, uint64_t count, double* total_out) {
     rc = r->prec == QVNT_F64 ? build_levels<double>(r, r->tree, count, info, true)
                              : build_levels<float>(r, r->tree, count, info, true);
     if (rc) return rc;
-    if (total_out) {
-        QVNT_HIP(hipMemcpyAsync(total_out, r->tree + info.off[info.top], sizeof(double), hipMemcpyDeviceToHost, r->stream));
-        QVNT_HIP(hipStreamSynchronize(r->stream));
+    HostBlock host(r->device, kHostSmall);
+    double* total_dev = host.p ? static_cast<double*>(host.p) : r->tree + info.off[info.top];
+    if (r->prec == QVNT_F64)
+        hipLaunchKernelGGL(k_total<double>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c64*>(r->psi),
+                           (const double*)r->tree, info, total_dev);
+    else
+        hipLaunchKernelGGL(k_total<float>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c32*>(r->psi),
+                           (const double*)r->tree, info, total_dev);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && !host.p) e = hipMemcpyAsync(total_out, total_dev, sizeof(double), hipMemcpyDeviceToHost, r->stream);
+    const hipError_t end = hipStreamSynchronize(r->stream);
+    if (e == hipSuccess) e = end;
+    if (e != hipSuccess) {
+        host.keep_out();
+        return fail(QVNT_E_HIP, std::string("norm: ") + hipGetErrorString(e));
     }
+    if (host.p) std::memcpy(total_out, host.p, sizeof(double));
     return QVNT_OK;
 }
 
@@ -379,14 +481,37 @@ int sample_launch(qvnt_reg* r, uint64_t count, const double* u_dev, size_t shots
     return sample_into(r, r->tree, count, u_dev, 0.0, shots, out_dev, total_dev, true);
 }
 
-// The outcomes land in iscratch[0, shots) and the total right after them
-// (iscratch holds shots_cap + 1 words), so one copy brings both back; a
-// single draw goes to the kernel by value.
+// The draws come from, and the outcomes and the total go to, one block of
+// pinned host memory that the kernel reads and writes itself, where the draws
+// fit one (HostBlock): a copy each way cost more than the draws (1024 shots,
+// whole call: 10 qubits 50 us with the copies, 26 without; 17 qubits 49 and
+// 33; the norm alone 23 and 12, 27 and 16).  Otherwise the outcomes
+// land in iscratch[0, shots) and the total right after them (iscratch holds
+// shots_cap + 1 words), so one copy brings both back.  A single draw goes to
+// the kernel by value.
 int tree_sample(qvnt_reg* r, uint64_t count, const double* u, size_t shots, uint64_t* out, double* total_out) {
     if (shots == 0) return fail(QVNT_E_ARG, "no draws");
-    int rc = ensure_workspace(r, tree_doubles(count), shots);
+    const bool small = (2 * shots + 1) * sizeof(uint64_t) <= kHostSmall;
+    HostBlock host(r->device, small ? kHostSmall : 0);
+    int rc = ensure_workspace(r, tree_doubles(count), host.p ? 1 : shots);
     if (rc) return rc;
     if (tree_doubles(count) > r->tree_cap) return fail(QVNT_E_ARG, "measurement tree workspace too small");
+    if (host.p) {
+        uint64_t* words = static_cast<uint64_t*>(host.p);   // outcomes, total, draws
+        double* total_dev = reinterpret_cast<double*>(words + shots);
+        double* draws = total_dev + 1;
+        if (shots > 1) std::memcpy(draws, u, shots * sizeof(double));
+        rc = sample_into(r, r->tree, count, shots > 1 ? draws : nullptr, shots > 1 ? 0.0 : u[0], shots, words, total_dev, true);
+        const hipError_t e = hipStreamSynchronize(r->stream);
+        if (rc == QVNT_OK && e != hipSuccess) rc = fail(QVNT_E_HIP, std::string("draws: ") + hipGetErrorString(e));
+        if (rc) {
+            host.keep_out();
+            return rc;
+        }
+        std::memcpy(out, words, shots * sizeof(uint64_t));
+        std::memcpy(total_out, total_dev, sizeof(double));
+        return QVNT_OK;
+    }
     const double* u_dev = nullptr;
     if (shots > 1) {
         QVNT_HIP(hipMemcpyAsync(r->dscratch + 1, u, shots * sizeof(double), hipMemcpyHostToDevice, r->stream));
@@ -395,13 +520,11 @@ int tree_sample(qvnt_reg* r, uint64_t count, const double* u, size_t shots, uint
     double* total_dev = reinterpret_cast<double*>(r->iscratch + shots);
     rc = sample_into(r, r->tree, count, u_dev, shots > 1 ? 0.0 : u[0], shots, r->iscratch, total_dev, true);
     if (rc) return rc;
-    uint64_t one[2];
-    std::vector<uint64_t> many(shots > 1 ? shots + 1 : 0);
-    uint64_t* host = shots > 1 ? many.data() : one;
-    QVNT_HIP(hipMemcpyAsync(host, r->iscratch, (shots + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, r->stream));
+    std::vector<uint64_t> words(shots + 1);
+    QVNT_HIP(hipMemcpyAsync(words.data(), r->iscratch, (shots + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, r->stream));
     QVNT_HIP(hipStreamSynchronize(r->stream));
-    std::memcpy(out, host, shots * sizeof(uint64_t));
-    std::memcpy(total_out, host + shots, sizeof(double));
+    std::memcpy(out, words.data(), shots * sizeof(uint64_t));
+    std::memcpy(total_out, words.data() + shots, sizeof(double));
     return QVNT_OK;
 }
 

@@ -45,6 +45,8 @@ struct DeviceCache {
     std::multimap<size_t, void*> blocks;  // by size
     size_t total = 0;
     std::vector<hipStream_t> streams;     // idle
+    std::multimap<size_t, void*> host;    // pinned host blocks, by size
+    size_t host_total = 0;
 };
 
 // Never destroyed: a register freed while the process exits (after this
@@ -116,6 +118,39 @@ void dev_release(int device, void* p, size_t bytes) {
         }
     }
     (void)hipFree(p);
+}
+
+HostBlock::HostBlock(int dev, size_t n) : device(dev), bytes(n) {
+    if (!bytes || !cached_device(device)) return;
+    {
+        DeviceCache& c = cache_of(device);
+        std::lock_guard<std::mutex> lk(c.mu);
+        auto it = c.host.find(bytes);
+        if (it != c.host.end()) {
+            p = it->second;
+            c.host_total -= bytes;
+            c.host.erase(it);
+            return;
+        }
+    }
+    OnDevice on(device);
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) == hipSuccess) return;
+    (void)hipGetLastError();
+    p = nullptr;
+}
+
+HostBlock::~HostBlock() {
+    if (!p) return;
+    DeviceCache& c = cache_of(device);
+    {
+        std::lock_guard<std::mutex> lk(c.mu);
+        if (c.host_total + bytes <= kHostTotal) {
+            c.host.emplace(bytes, p);
+            c.host_total += bytes;
+            return;
+        }
+    }
+    (void)hipHostFree(p);
 }
 
 int stream_acquire(int device, hipStream_t* s) {
@@ -208,6 +243,9 @@ int qvnt_cache_trim(void) {
         std::lock_guard<std::mutex> lk(c.mu);
         for (hipStream_t s : c.streams) (void)hipStreamDestroy(s);
         c.streams.clear();
+        for (auto& kv : c.host) (void)hipHostFree(kv.second);
+        c.host.clear();
+        c.host_total = 0;
     }
     return QVNT_OK;
 }

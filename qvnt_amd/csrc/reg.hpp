@@ -75,6 +75,24 @@ constexpr size_t kCacheBlock = size_t(64) << 20;
 constexpr size_t kCacheTotal = size_t(256) << 20;
 int dev_alloc(int device, void** p, size_t bytes);
 void dev_release(int device, void* p, size_t bytes);
+// HostBlock: a block of exactly `bytes` of pinned host memory for one call,
+// that kernels read and write directly; p is null when there is none (0
+// bytes, or the allocation failed).  The blocks are cached per device like the
+// others, at most kHostTotal of them.  The owner's stream is synchronized
+// before it ends, or, where that failed, keep_out() keeps the block from
+// being used again.
+constexpr size_t kHostSmall = size_t(64) << 10;
+constexpr size_t kHostTotal = size_t(32) << 20;
+struct HostBlock {
+    int device;
+    size_t bytes;
+    void* p = nullptr;
+    HostBlock(int device, size_t bytes);
+    ~HostBlock();
+    HostBlock(const HostBlock&) = delete;
+    HostBlock& operator=(const HostBlock&) = delete;
+    void keep_out() { p = nullptr; }
+};
 int stream_acquire(int device, hipStream_t* s);
 void stream_release(int device, hipStream_t s);
 
