@@ -575,7 +575,19 @@ int rescale(qvnt_reg* r, double scale) {
 }
 
 int probabilities(qvnt_reg* r, double inv_total, double* dst, uint64_t n) {
-    // bounded device staging: chunks of up to 2^24 probabilities
+    const int done = read_back(r, dst, n * sizeof(double), [&](void* block, size_t off, size_t bytes) {
+        const uint64_t first = off / sizeof(double), m = bytes / sizeof(double);
+        const dim3 grid((unsigned)((m + kBlock - 1) / kBlock));
+        if (r->prec == QVNT_F64)
+            hipLaunchKernelGGL(k_probs<double>, grid, dim3(kBlock), 0, r->stream, static_cast<const c64*>(r->psi) + first, m, inv_total,
+                               static_cast<double*>(block));
+        else
+            hipLaunchKernelGGL(k_probs<float>, grid, dim3(kBlock), 0, r->stream, static_cast<const c32*>(r->psi) + first, m, inv_total,
+                               static_cast<double*>(block));
+        return hipGetLastError();
+    });
+    if (done != kNoBlock) return done;
+    // no pinned memory: bounded device staging: chunks of up to 2^24 probabilities
     const uint64_t chunk = n < (1ull << 24) ? n : (1ull << 24);
     void* vbuf = nullptr;
     if (dev_alloc(r->device, &vbuf, chunk * sizeof(double)) != QVNT_OK)

@@ -227,6 +227,13 @@ int check_device(int* dev) {
     return QVNT_OK;
 }
 
+// Device memory to pinned host memory, 16 bytes a thread (a state is at least
+// 64 bytes, and a power of two).
+__global__ __launch_bounds__(256) void k_read(const uint4* __restrict__ from, uint4* __restrict__ to, uint64_t words) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i < words) to[i] = from[i];
+}
+
 int check_reg(const qvnt_reg* r) { return r ? QVNT_OK : fail(QVNT_E_ARG, "null register"); }
 
 }  // namespace
@@ -429,6 +436,14 @@ int qvnt_reg_compare(qvnt_reg* a, qvnt_reg* b, double out[5]) {
 int qvnt_reg_get_state(qvnt_reg* r, void* dst, size_t bytes) {
     if (int rc = check_reg(r)) return rc;
     if (!dst || bytes != r->len * r->amp_bytes()) return fail(QVNT_E_ARG, "state copy needs len * amplitude bytes");
+    const int rc = read_back(r, dst, bytes, [&](void* block, size_t off, size_t n) {
+        // (a kernel of ours: the runtime's copies queue 10 us apart)
+        const uint64_t words = n / sizeof(uint4);
+        hipLaunchKernelGGL(k_read, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, r->stream,
+                           reinterpret_cast<const uint4*>(static_cast<const unsigned char*>(r->psi) + off), static_cast<uint4*>(block), words);
+        return hipGetLastError();
+    });
+    if (rc != kNoBlock) return rc;
     QVNT_HIP(hipMemcpyAsync(dst, r->psi, bytes, hipMemcpyDeviceToHost, r->stream));
     QVNT_HIP(hipStreamSynchronize(r->stream));
     return QVNT_OK;
