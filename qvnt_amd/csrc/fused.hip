@@ -479,15 +479,21 @@ __device__ __forceinline__ uint64_t global_offset(const uint32_t* tp, uint32_t l
 // registers run over, and the thread's address.
 template <class R>
 struct Edge {
+    bool own;
     uint32_t pos[kRegBits];
     uint32_t tb;              // local index of register 0
     uint64_t step[kRegBits];  // global offsets of the register bits (uniform)
-    // own: in the layout of phase ph, else with the tile's top bits in the registers
-    __device__ __forceinline__ void set(const FPass& pass, const FPhase& ph, bool own, uint32_t tid) {
+    // The first (e 0) or last (1) phase's own layout where a whole 128-byte
+    // line stays among the threads in it (local bits 0..2 in FP64, 0..3 in
+    // FP32; saves one exchange), else the tile's top bits in the registers.
+    __device__ __forceinline__ void set(const FPass& pass, int e, bool allow, uint32_t tid) {
+        own = allow && !pass.edge_dense[e] && (pass.edge[e] & 63u) >= (sizeof(R) == 8 ? 3u : 4u);
+        const uint32_t l = own ? pass.edge[e] : (pass.t - kRegBits) * 0x01010101u + 0x03020100u;
+        const uint32_t g = own ? pass.edge_global[e] : pass.top_global;
 #pragma unroll
         for (int j = 0; j < kRegBits; ++j) {
-            pos[j] = own ? ph.rpos[j] : pass.t - kRegBits + j;
-            step[j] = 1ull << pass.tpos[pos[j]];
+            pos[j] = (l >> (8 * j)) & 63u;
+            step[j] = 1ull << ((g >> (8 * j)) & 63u);
         }
         tb = spread<kRegBits>(tid, pos);
     }
@@ -500,34 +506,28 @@ struct Edge {
     }
 };
 
-// Whether a tile can be read or written in the phase's own layout: a whole
-// 128-byte line has to stay among the threads (local bits 0..2 in FP64, 0..3
-// in FP32).  Saves one exchange.
-template <class R>
-__device__ __forceinline__ bool edge_layout(const FPhase& ph) {
-    return !ph.dense && ph.rpos[0] >= (sizeof(R) == 8 ? 3u : 4u);
-}
-
 // Passes of at most this many tiles bring their program near first
 // (warm_program).  With more, the blocks before have done so, and the touches
 // only take time: 31-qubit Ising steps in FP32 96 ms without, 112 with.
 constexpr uint32_t kWarmTiles = 2048;
 
-// Brings the pass's ops and coefficients into the L2 of this block's XCD:
-// thread k touches op k and its coefficient lines, all at once, where the op
+// Brings the pass's phases, ops and coefficients into the L2 of this block's
+// XCD: one load a line, all at once and beside the tile's own, where the op
 // loop's scalar loads would wait for memory one after the other (16 qubits
-// FP64, 400 gates: 370 us of k_fused without, 250 with).
-__device__ __forceinline__ uint32_t warm_program(const FOp* __restrict__ ops, const double* __restrict__ coef, uint32_t begin,
-                                                 uint32_t end, uint32_t tid, uint32_t nth) {
+// FP64, 400 gates: 370 us of k_fused without; with the ops' tables found
+// through the ops, and the edges' layouts through the phases, three misses
+// one after the other before the first op, 240; 216 so).
+__device__ __forceinline__ uint32_t warm_program(const FPass& pass, const FPhase* __restrict__ phases, const FOp* __restrict__ ops,
+                                                 const double* __restrict__ coef, uint32_t tid) {
     uint32_t seen = 0;
-    for (uint32_t o = begin + tid; o < end; o += nth) {
-        const FOp& op = ops[o];
-        const uint32_t type = op.type, c = op.coef;
-        const bool outside = ((uint64_t)(op.la | op.lb) | op.ga | op.gb) != 0;
-        const uint32_t n = type == OP_S ? 72u : type == OP_G ? 128u : type == OP_D ? (outside ? 128u : 32u) : type == OP_M4 ? 32u : type == OP_P4 ? 16u
-                           : type == OP_M2 || type == OP_P4R ? 8u : type == OP_A2 ? 4u : 0u;
-        for (uint32_t k = 0; k < n; k += 16u) seen ^= reinterpret_cast<const uint32_t*>(coef + c + k)[0];
-    }
+    const auto touch = [&](const void* from, const void* to) {
+        const unsigned char* p = static_cast<const unsigned char*>(from);
+        for (uint32_t k = tid * 128u; k < (uint32_t)(static_cast<const unsigned char*>(to) - p); k += pass.nthreads * 128u)
+            seen ^= *reinterpret_cast<const uint32_t*>(p + k);
+    };
+    touch(ops + pass.op_begin, ops + pass.op_end);
+    touch(coef + pass.coef_begin, coef + pass.coef_end);
+    touch(phases + pass.phase_begin, phases + pass.phase_end);
     return seen;
 }
 
@@ -542,17 +542,21 @@ template <class R, bool GATED = false>
 __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPass& pass, const FPhase* __restrict__ phases,
                                            const FOp* __restrict__ ops, const double* __restrict__ coef,
                                            uint64_t tile_index, uint32_t tiles, R* lds, uint32_t tid, bool active = true) {
+    const bool warm = tiles <= kWarmTiles;
+    uint32_t seen = 0;
+    if (warm) seen = warm_program(pass, phases, ops, coef, tid);
     uint32_t tp[kMaxTile];
     load_tpos(pass, tp);
     const uint64_t tile = tile_base(tp, pass.t, tile_index);
     const uint32_t p0 = pass.phase_begin, p1 = pass.phase_end;
     cplx<R> v[kRegs];
-    const bool own_in = edge_layout<R>(phases[p0]);
+    bool own_in;
     uint32_t tb;
     Layout cur;
     {
         Edge<R> in;
-        in.set(pass, phases[p0], own_in, tid);
+        in.set(pass, 0, true, tid);
+        own_in = in.own;
         tb = in.tb;
         cur = layout_of<kRegBits>(tb, in.pos);
         const cplx<R>* p = psi + (tile | global_offset(tp, tb));
@@ -565,13 +569,13 @@ __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPas
             }
         }
     }
-    if (tiles <= kWarmTiles) {
-        const uint32_t seen = warm_program(ops, coef, phases[p0].op_begin, phases[p1 - 1].op_end, tid, pass.nthreads);
-        asm volatile("" ::"v"(seen));
-    }
-    FOp next = ops[phases[p0].op_begin];
+    if (warm) asm volatile("" ::"v"(seen));
+    // (each phase's header, too, is loaded while the one before runs)
+    FOp next = ops[pass.op_begin];
+    FPhase ahead = phases[p0];
     for (uint32_t p = p0; p < p1; ++p) {
-        const FPhase& ph = phases[p];
+        const FPhase ph = ahead;
+        ahead = phases[p + 1];
         if (ph.dense) {
             const Layout to = dense_layout(ph, tid);
             exchange<kRegBits>(v, lds, cur, to);
@@ -587,18 +591,18 @@ __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPas
         }
         run_phase(v, ph.op_begin, ph.op_end, ops, coef, tb, tile, next);
     }
-    const FPhase& last = phases[p1 - 1];
-    const bool own_out = edge_layout<R>(last) && !pass.permuted;
     Edge<R> out;
-    out.set(pass, last, own_out, tid);
+    out.set(pass, 1, !pass.permuted, tid);
     if (pass.permuted) {
         // through the pass's qubit permutation: the thread that stores local
         // index tid + j 2^(t-4) reads it from pimg / pout
         uint32_t s = 0;
-        for (uint32_t k = 0; k + kRegBits < pass.t; ++k) s ^= unswizzled(pass.pimg[k]) & (0u - ((tid >> k) & 1u));
+#pragma unroll
+        for (uint32_t k = 0; k < (uint32_t)(kMaxTile - kRegBits); ++k)
+            if (k + kRegBits < pass.t) s ^= unswizzled(pass.pimg[k]) & (0u - ((tid >> k) & 1u));
         s = swz(s);
         exchange<kRegBits>(v, lds, cur, [&](int i) { return s ^ swz(unswizzled(pass.pout[i])); });
-    } else if (!own_out && !pass.direct_last) {
+    } else if (!out.own && !pass.direct_last) {
         exchange<kRegBits>(v, lds, cur, layout_of<kRegBits>(out.tb, out.pos));
     }
     if (!GATED || active) {

@@ -1234,6 +1234,8 @@ void compile_pass(Program& prog, const PassPlan& pp_in, unsigned dense_min) {
     relocate_diagonals(plans, fp);
 
     fp.phase_begin = (uint32_t)prog.phases.size();
+    fp.op_begin = (uint32_t)prog.ops.size();
+    fp.coef_begin = (uint32_t)prog.coef.size();
     for (PhasePlan& plan : plans) {
         if (plan.prims.empty() && plans.size() > 1) continue;  // its diagonals all moved
         const uint32_t Rl = plan.Rl;
@@ -1367,6 +1369,17 @@ void compile_pass(Program& prog, const PassPlan& pp_in, unsigned dense_min) {
         prog.phases.push_back(ph);
     }
     fp.phase_end = (uint32_t)prog.phases.size();
+    fp.op_end = (uint32_t)prog.ops.size();
+    fp.coef_end = (uint32_t)prog.coef.size();
+    for (int k = 0; k < kRegBits; ++k) {
+        for (int e = 0; e < 2; ++e) {
+            const FPhase& ph = prog.phases[e ? fp.phase_end - 1 : fp.phase_begin];
+            fp.edge[e] |= ph.rpos[k] << (8 * k);
+            fp.edge_global[e] |= fp.tpos[ph.rpos[k]] << (8 * k);
+            fp.edge_dense[e] = ph.dense;
+        }
+        fp.top_global |= fp.tpos[fp.t - kRegBits + k] << (8 * k);
+    }
     auto is_top = [&](const FPhase& ph) {
         if (ph.dense) return false;  // dense phases work from the LDS tile
         for (int k = 0; k < kRegBits; ++k)
@@ -1407,6 +1420,10 @@ void append_program(Program& dst, const Program& src) {
     for (FPass fp : src.passes) {
         fp.phase_begin += pb;
         fp.phase_end += pb;
+        fp.op_begin += ob;
+        fp.op_end += ob;
+        fp.coef_begin += cb;
+        fp.coef_end += cb;
         dst.passes.push_back(fp);
     }
     for (FPhase ph : src.phases) {

@@ -133,6 +133,12 @@ struct FPass {
     // tpos again, one byte each (byte k of the 16 = tpos[k], 0 past t):
     // four scalar registers for the kernel's loops over the local bits
     uint32_t tpack[4];
+    // What the kernel needs before it can read the tile, beside the pass's
+    // other fields: the register bits of the first and last phase, one byte
+    // each, local and global, and whether they are dense; the global positions
+    // of local bits t-4..t-1; and where the pass's ops and coefficients lie.
+    uint32_t edge[2], edge_global[2], edge_dense[2], top_global;
+    uint32_t op_begin, op_end, coef_begin, coef_end;
 };
 
 // One register's pass in a batched launch: byte offsets into the program
