@@ -646,29 +646,21 @@ __global__ QVNT_FUSED_BOUNDS void k_fused(cplx<R>* __restrict__ psi, FPass pass,
 }
 
 // The batched form: the tiles of one pass of many registers in one launch
-// (every item's pass has the launch's t).  Block b (in XCD order,
-// xcd_order) runs batch_tiles tiles of item map[b], from tile
-// (b - items[map[b]].block0) * batch_tiles, one after the other; registers,
-// passes and programs are addressed by offsets from the two base pointers.
+// (every item's pass has the launch's t).  Block b (in XCD order, xcd_order)
+// runs tile b - items[map[b]].block0 of item map[b]; registers, passes and
+// programs are addressed by offsets from the two base pointers.  (Two tiles a
+// block share what the scalar cache holds of the program, which paid with two
+// waves per SIMD; with four, 4096 registers FP64 take 30.6 ms with two tiles
+// a block and 29.3 with one.)
 template <class R>
 __global__ QVNT_FUSED_BOUNDS void k_batch(cplx<R>* __restrict__ arena, const unsigned char* __restrict__ prog,
                                                const BItem* __restrict__ items, const uint32_t* __restrict__ map) {
     extern __shared__ unsigned char smem[];
     const uint32_t b = xcd_order(blockIdx.x, gridDim.x);
     const BItem it = items[map[b]];
-    const FPass& pass = *reinterpret_cast<const FPass*>(prog + it.pass_off);
-    constexpr uint32_t per_block = batch_tiles(sizeof(R) == 8);
-    const uint32_t first = (b - it.block0) * per_block;
-    for (uint32_t k = 0; k < per_block; ++k) {
-        const uint32_t tile = first + k;
-        if (tile >= it.tiles) break;  // uniform
-        // the tile's first LDS writes may hit elements other threads still
-        // read in the previous tile's last phase
-        if (k) __syncthreads();
-        fused_tile<R>(arena + it.psi_off, pass, reinterpret_cast<const FPhase*>(prog + it.phase_off),
-                      reinterpret_cast<const FOp*>(prog + it.op_off), reinterpret_cast<const double*>(prog + it.coef_off), tile,
-                      k ? ~0u : it.tiles, reinterpret_cast<R*>(smem), threadIdx.x);
-    }
+    fused_tile<R>(arena + it.psi_off, *reinterpret_cast<const FPass*>(prog + it.pass_off),
+                  reinterpret_cast<const FPhase*>(prog + it.phase_off), reinterpret_cast<const FOp*>(prog + it.op_off),
+                  reinterpret_cast<const double*>(prog + it.coef_off), b - it.block0, it.tiles, reinterpret_cast<R*>(smem), threadIdx.x);
 }
 
 // One work unit of the persistent batched kernel (below): up to
