@@ -175,7 +175,8 @@ int qvnt_reg_with_state(uint32_t q_num, uint64_t state, qvnt_prec prec, qvnt_reg
  * allocation that fails empties the device's block cache and tries once
  * more. */
 int qvnt_reg_free(qvnt_reg* reg);
-/* Frees every cached block and idle stream of every device.  No counterpart
+/* Frees every cached block (device memory, and the pinned host blocks that
+ * results come back through) and idle stream of every device.  No counterpart
  * in the reference (it keeps no cache): for callers that share the GPU's
  * memory with another allocator and want the cache's memory back. */
 int qvnt_cache_trim(void);
