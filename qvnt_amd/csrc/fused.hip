@@ -560,13 +560,19 @@ __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPas
         tb = in.tb;
         cur = layout_of<kRegBits>(tb, in.pos);
         const cplx<R>* p = psi + (tile | global_offset(tp, tb));
+        // One branch around the 16 loads: with a branch each (uniform ones
+        // stay branches in this file) every load waited for the one before
+        // it.  k_batch_persist, 1024 registers of 10..20 qubits, FP32, tiles
+        // of 12: 11.1 ms so, 8.9 now; FP64 12.2 and 10.4.
+        if (!GATED || active) {
 #pragma unroll
-        for (int i = 0; i < kRegs; ++i) {
-            v[i] = cplx<R>{(R)0, (R)0};
-            if (!GATED || active) {
+            for (int i = 0; i < kRegs; ++i) {
                 const cplx<R>* q = p + in.off(i);
                 v[i] = cplx<R>{__builtin_nontemporal_load(&q->re), __builtin_nontemporal_load(&q->im)};
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kRegs; ++i) v[i] = cplx<R>{(R)0, (R)0};
         }
     }
     if (warm) asm volatile("" ::"v"(seen));
