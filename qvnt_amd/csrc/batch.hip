@@ -12,6 +12,7 @@
 // own registers of that size.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <new>
@@ -209,6 +210,19 @@ void compile_plans(const std::vector<std::vector<qvnt_gate>>& gates, const std::
     *bad = err.load();
 }
 
+// Blocks of the persistent kernel for rounds of `phases` phases in all: B
+// blocks run them in phases * 6.5 us / B and meet at a barrier of B * 0.16 us,
+// least in sum at B = sqrt(40 phases); no more than are resident.  With as
+// many as 12 waves a CU allow, always, 64 registers of 16 qubits FP64 with
+// tiles of 10 took 2.54 ms (3072 blocks), so 0.87 (488); with tiles of 12 0.62
+// (768) and 0.50 (328); 1024 registers of 10..20 qubits FP32 with tiles of 13
+// 12.3 (256) and 7.6 (512, two a CU), with tiles of 12 8.9 (768) and 7.6
+// (1280).  sqrt(25 phases) and sqrt(55 phases) differ from it by up to 14 %
+// and 4 %.
+uint32_t persist_blocks(double phases) {
+    return (uint32_t)std::min(1e9, std::max(8.0, std::sqrt(40.0 * phases)));
+}
+
 // Packs the plans of `sel` and builds their rounds.
 int build_schedule(qvnt_batch* b, const std::vector<RegPlan>& plans, const std::vector<uint32_t>& sel, Schedule& S) {
     S.release();
@@ -243,6 +257,7 @@ int build_schedule(qvnt_batch* b, const std::vector<RegPlan>& plans, const std::
     std::vector<BItem> p_items;
     std::vector<PUnit> p_units;
     std::vector<uint32_t> p_rounds(1, 0);
+    double p_phases = 0.0;   // phases that the units run, one after the other
     std::vector<unsigned char> lhost;
     for (uint32_t r = 0; r < S.rounds; ++r) {
         std::map<uint32_t, std::vector<uint32_t>> by_t;
@@ -268,6 +283,7 @@ int build_schedule(qvnt_batch* b, const std::vector<RegPlan>& plans, const std::
                 map.insert(map.end(), tiles, (uint32_t)items.size());
                 items.push_back(it);
                 const uint64_t per_unit = 1ull << (S.tmax - fp.t);
+                p_phases += (double)((tiles + per_unit - 1) / per_unit) * (fp.phase_end - fp.phase_begin);
                 for (uint64_t j = 0; j < tiles; j += per_unit)
                     p_units.push_back(PUnit{(uint32_t)p_items.size(), (uint32_t)j, (uint32_t)std::min(tiles, j + per_unit), 0u});
                 p_items.push_back(it);
@@ -295,7 +311,7 @@ int build_schedule(qvnt_batch* b, const std::vector<RegPlan>& plans, const std::
     for (uint32_t r = 0; r < S.rounds; ++r) widest = std::max(widest, p_rounds[r + 1] - p_rounds[r]);
     uint32_t resident = 0;
     if (S.tmax >= (uint32_t)qvnt::fusion::kMinFused && qvnt::batch_persist_grid(b->prec, S.tmax, &resident) == QVNT_OK) {
-        S.persist_blocks = std::min(resident, widest);
+        S.persist_blocks = std::min({resident, widest, persist_blocks(p_phases / S.rounds)});
         // a multiple of 8: every XCD gets as many blocks (k_batch_persist
         // hands each XCD its own range of a round's units)
         if (S.persist_blocks >= 8) S.persist_blocks &= ~7u;

@@ -825,10 +825,6 @@ int batch_persist_grid(qvnt_prec prec, uint32_t tmax, uint32_t* blocks) {
     else
         QVNT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch_persist<float>, threads, lds));
     if (per_cu <= 0) return fail(QVNT_E_HIP, "the persistent batched kernel does not fit a compute unit");
-    // three waves per SIMD (QVNT_PERSIST_BOUNDS): more resident blocks only
-    // lengthen the grid barriers
-    const int most = 12 / (threads < 64 ? 1 : threads / 64);
-    if (per_cu > most && most > 0) per_cu = most;
     *blocks = (uint32_t)per_cu * (uint32_t)cus;
     return QVNT_OK;
 }
