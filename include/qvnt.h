@@ -252,7 +252,8 @@ int qvnt_reg_sample_mask_noalloc(qvnt_reg* reg, uint64_t mask, const double* u, 
 int qvnt_reg_compare(qvnt_reg* a, qvnt_reg* b, double out[5]);
 
 /* Copy-out / copy-in of the interleaved amplitudes (bytes = len * 2 *
- * sizeof(double or float)).  Blocking. */
+ * sizeof(double or float)).  Blocking.  Into pinned or device memory a state
+ * goes with one copy. */
 int qvnt_reg_get_state(qvnt_reg* reg, void* dst, size_t bytes);
 int qvnt_reg_set_state(qvnt_reg* reg, const void* src, size_t bytes);
 /* Debug of QReg (quant.rs:603-623): "QReg { 0: Complex { re: 0.25, im: 0.0 },

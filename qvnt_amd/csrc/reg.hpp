@@ -97,6 +97,13 @@ struct HostBlock {
 int stream_acquire(int device, hipStream_t* s);
 void stream_release(int device, hipStream_t s);
 
+// Where the caller's destination lies.  Device memory (managed memory with
+// it) takes a copy of the runtime's, as no host thread may write it; pinned
+// memory the same, from the size on where one copy over the bus beats the ring
+// below and its second copy by a host thread.
+enum class Memory { Pageable, Pinned, Device };
+Memory memory_of(const void* p);
+
 // `bytes` of results from the register's stream to pageable memory:
 // fill(block, offset, n) enqueues the next n of them into a pinned block.
 // Several blocks, so that one is copied to dst while the next ones fill.  The runtime's
