@@ -397,7 +397,8 @@ int ensure_workspace(qvnt_reg* r, size_t tree_doubles, size_t shots) {
 
 // The stored levels of the first `count` weights into `tree` (laid out by
 // tree_info(count)); timed: bracket the launches with the register's timing
-// events (the allocation-free path passes false: it creates no events).
+// events (the allocation-free path passes false: it creates no events, and so
+// does the norm, which brackets its last kernel with them).
 template <class R>
 int build_levels(qvnt_reg* r, double* tree, uint64_t count, const TreeInfo& info, bool timed) {
     if (info.top <= kLeafLog) return QVNT_OK;  // the leaves are the level below the top
@@ -448,18 +449,23 @@ int tree_build(qvnt_reg* r, uint64_t count, double* total_out) {
     const TreeInfo info = tree_info(count);
     int rc = ensure_workspace(r, (size_t)(info.off[info.top] + 1), 1);
     if (rc) return rc;
-    rc = r->prec == QVNT_F64 ? build_levels<double>(r, r->tree, count, info, true)
-                             : build_levels<float>(r, r->tree, count, info, true);
-    if (rc) return rc;
     HostBlock host(r->device, kHostSmall);
     double* total_dev = host.p ? static_cast<double*>(host.p) : r->tree + info.off[info.top];
-    if (r->prec == QVNT_F64)
-        hipLaunchKernelGGL(k_total<double>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c64*>(r->psi),
-                           (const double*)r->tree, info, total_dev);
-    else
-        hipLaunchKernelGGL(k_total<float>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c32*>(r->psi),
-                           (const double*)r->tree, info, total_dev);
-    hipError_t e = hipGetLastError();
+    hipError_t e = hipSuccess;
+    {
+        // (one reduction in the statistics: the stored levels, if any, and the root)
+        Timed t(r, QVNT_K_REDUCE, (double)r->amp_bytes() * (double)count);
+        rc = r->prec == QVNT_F64 ? build_levels<double>(r, r->tree, count, info, false)
+                                 : build_levels<float>(r, r->tree, count, info, false);
+        if (rc) return rc;
+        if (r->prec == QVNT_F64)
+            hipLaunchKernelGGL(k_total<double>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c64*>(r->psi),
+                               (const double*)r->tree, info, total_dev);
+        else
+            hipLaunchKernelGGL(k_total<float>, dim3(1), dim3(kWave), 0, r->stream, static_cast<const c32*>(r->psi),
+                               (const double*)r->tree, info, total_dev);
+        e = hipGetLastError();
+    }
     if (e == hipSuccess && !host.p) e = hipMemcpyAsync(total_out, total_dev, sizeof(double), hipMemcpyDeviceToHost, r->stream);
     const hipError_t end = hipStreamSynchronize(r->stream);
     if (e == hipSuccess) e = end;
