@@ -142,13 +142,15 @@ HostBlock::HostBlock(int dev, size_t n) : device(dev), bytes(n) {
 HostBlock::~HostBlock() {
     if (!p) return;
     DeviceCache& c = cache_of(device);
-    {
+    try {
         std::lock_guard<std::mutex> lk(c.mu);
         if (c.host_total + bytes <= kHostTotal) {
             c.host.emplace(bytes, p);
             c.host_total += bytes;
             return;
         }
+    } catch (const std::bad_alloc&) {
+        // (no memory to remember the block in)
     }
     (void)hipHostFree(p);
 }
