@@ -93,7 +93,8 @@ struct Run {
     ROut outer[kMaxOps];
     ROp op[kMaxOps];
 };
-static_assert(sizeof(Run) <= 4096, "a run is passed as kernel arguments");
+// (16 bytes: the launch's other arguments, psi and tiles)
+static_assert(sizeof(Run) + 16 <= 4096, "a run is passed as kernel arguments");
 
 // The next step of a plain apply of a validated queue on 2^ns amplitudes.
 // Done: nothing is left.  RunStep: gates [from, from + count) as `run`.
