@@ -21,6 +21,10 @@ struct Prim {
 };
 
 constexpr size_t kMaxPrims = 64;
+// From here on a queue's runs are weighed (Cost); below, a launch takes longer
+// than a pass, and two SingleOps are a run (18 qubits FP64: 3 gates with 1
+// control 4.8 us as a run, 10.9 alone; 20 with a control each 6.1 and 8.6).
+constexpr unsigned kWeighedQubits = 20;
 
 uint64_t low_bit(uint64_t x) { return x & (~x + 1); }
 
@@ -92,6 +96,33 @@ unsigned single_share(const qvnt_gate& g, unsigned ns, bool fp64) {
     return halves < 6 ? 64u >> halves : 1u;
 }
 
+// What single kernels and a run take, in 1/64ths of a pass over the state
+// (read and written at 6 TB/s).  Fitted to queues of 2 to 70 x, ry and rz with
+// 0 to 6 controls, on the top qubits and in the tile, on 20 to 28 qubits in
+// both precisions, each timed all as runs and all as single kernels (1248
+// pairs): the choice takes 0.1 % longer than the better of the two on average,
+// a third at most (26 qubits FP32, 70 x with 6 controls each, left single).
+struct Cost {
+    unsigned ns;
+    bool fp64;
+    double launch;
+    Cost(unsigned n, bool f64)
+        // 5.6 us from one kernel to the next
+        : ns(n), fp64(f64), launch(5.6 * 64.0 * 6.0e6 / (double)((f64 ? 32ull : 16ull) << n)) {}
+    double single(unsigned share) const { return share > launch / 2.0 ? share + launch / 2.0 : launch; }
+    // An op's arithmetic: 28 qubits FP32 20 ry in 1.69 ms (a pass 0.77), 40 with
+    // 4 controls in 3.27, with 5 in 2.11; 25 qubits, where each block has one
+    // tile, 0.29 and 0.17 (0.09); FP64 28 qubits 1.70 for 20 and 2.21 for 40
+    // (1.59).  Moves (x, swap): 40 with 4 controls FP32 1.52.
+    double op(bool move, unsigned share) const {
+        if (fp64) return move ? 0.7 : 1.4;
+        if (move) return 1.7;
+        const double most = ns <= 25 ? 5.0 : 6.3, part = 2.0 + (ns <= 25 ? 0.6 : 0.8) * share;
+        return part < most ? part : most;
+    }
+    double run(double ops) const { return (ops + 20.0 > 70.0 ? ops + 20.0 : 70.0) + launch; }
+};
+
 }  // namespace
 
 Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, unsigned regs, unsigned max_tile, Run* run) {
@@ -109,16 +140,29 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, uns
     const unsigned tmax = ns < max_tile ? ns : max_tile;
     const unsigned rows = row_bits(fp64) + regs < tmax ? row_bits(fp64) : tmax - regs;
 
-    // the longest prefix of the queue that fits: its tile qubits, and its
-    // phases' register qubits
+    // The longest prefix of the queue that fits: its tile qubits, and its
+    // phases' register qubits.  Where a pass takes longer than a launch, the
+    // prefix that gains most over its gates' own kernels, if any does.  (By
+    // the bytes alone, more than 1.25 passes' worth, gates with many controls
+    // went into FP32 runs that took longer: 28 qubits, 20 ry with 4 controls
+    // in the tile 1.70 ms as a run and 1.10 alone, 40 of them 3.27 and 2.19, 40
+    // with 5 controls 2.11 and 1.57.)
+    const Cost cost(ns, fp64);
+    const bool weigh = ns >= kWeighedQubits;
+    double alone = 0.0, ops = 0.0, best_gain = 0.0;
+    struct Prefix {
+        unsigned count, phases;
+        uint64_t tile, mixed;   // mixed: of its last phase
+        size_t last;
+    } best{0, 0, 0, 0, 0};
     Prim list[kMaxOps];
     uint64_t mixed[kMaxPhases];
     unsigned ends[kMaxPhases];
-    unsigned count = 0, phases = 1, share = 0;
+    unsigned count = 0, phases = 1;
     uint64_t tile = (1ull << rows) - 1u;
     mixed[0] = 0;
-    size_t i = *pos, last = *pos, gates = 0;
-    for (; i < n; ++i) {
+    size_t gates = 0;
+    for (size_t i = *pos; i < n; ++i) {
         const int k = lower(g[i], ns, prims);
         if (k < 0) break;
         if (k == 0) continue;
@@ -152,20 +196,29 @@ Step next(const qvnt_gate* g, size_t n, size_t* pos, unsigned ns, bool fp64, uns
         count = c2;
         phases = ph2;
         tile = t2;
-        share += single_share(g[i], ns, fp64);
         ++gates;
-        last = i + 1;
+        const unsigned share = single_share(g[i], ns, fp64);
+        alone += cost.single(share);
+        for (int j = 0; j < k; ++j) ops += cost.op(prims[j].family == F_X || prims[j].family == F_SWAP, share);
+        const double gain = alone - cost.run(ops);
+        // (one SingleOp alone is its own kernel's work)
+        if (gates >= 2 && (!weigh || gain >= best_gain)) {
+            best_gain = gain;
+            best = {count, phases, tile, r2, i + 1};
+        }
     }
-    ends[phases - 1] = count;
-    // One SingleOp alone is its own kernel's work.  Where a pass takes longer
-    // than a launch, a run has to replace more than one pass over the state.
-    if (gates < 2 || (ns >= 20 && share < 80)) {
+    if (best.last == 0) {
         ++*pos;
         return step;
     }
+    count = best.count;
+    phases = best.phases;
+    tile = best.tile;
+    mixed[phases - 1] = best.mixed;
+    ends[phases - 1] = count;
     step.kind = Kind::RunStep;
-    step.count = last - step.from;
-    *pos = last;
+    step.count = best.last - step.from;
+    *pos = best.last;
 
     // the tile, filled with the lowest qubits
     for (unsigned q = 0; popc(tile) < tmax; ++q) tile |= 1ull << q;
