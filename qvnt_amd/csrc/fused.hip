@@ -178,22 +178,22 @@ __device__ __forceinline__ void apply_d(cplx<R>* v, const double* __restrict__ c
     for (int i = 0; i < kRegs; ++i) put<M>(v[i], mul_c(ld_coef<R>(c, i), v[i]), on);
 }
 // The same from a table of the lane's own: the phases are loaded before the
-// first is used, 16 of them in FP32 and 8 in FP64, where no more registers are
-// free.  (One at a time each waited for memory: k_fused of a 28-qubit QFT FP32
+// first is used, AHEAD at a time: 16 in FP32; 8 in FP64, where no more
+// registers are free, and in the persistent kernel, where 16 take FP32 from 92
+// registers and five waves a SIMD to 118 and four.  (One at a time each waited for memory: k_fused of a 28-qubit QFT FP32
 // 12.9 ms so, 11.9 now; of 15 random gates on 26 qubits 327 and 251 us; FP64
 // 16 qubits QFT 72 and 65 us.)
-template <bool M, class R>
+template <int AHEAD, bool M, class R>
 __device__ __forceinline__ void apply_d_lane(cplx<R>* v, const double* __restrict__ c, bool on) {
-    constexpr int kAhead = sizeof(R) == 8 ? 8 : 16;
 #pragma unroll
-    for (int i = 0; i < kRegs; i += kAhead) {
-        cplx<double> d[kAhead];
+    for (int i = 0; i < kRegs; i += AHEAD) {
+        cplx<double> d[AHEAD];
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) d[k] = cplx<double>{c[2 * (i + k)], c[2 * (i + k) + 1]};
+        for (int k = 0; k < AHEAD; ++k) d[k] = cplx<double>{c[2 * (i + k)], c[2 * (i + k) + 1]};
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) asm volatile("" : "+v"(d[k].re), "+v"(d[k].im));
+        for (int k = 0; k < AHEAD; ++k) asm volatile("" : "+v"(d[k].re), "+v"(d[k].im));
 #pragma unroll
-        for (int k = 0; k < kAhead; ++k) put<M>(v[i + k], mul_c(cplx<R>{(R)d[k].re, (R)d[k].im}, v[i + k]), on);
+        for (int k = 0; k < AHEAD; ++k) put<M>(v[i + k], mul_c(cplx<R>{(R)d[k].re, (R)d[k].im}, v[i + k]), on);
     }
 }
 
@@ -317,7 +317,7 @@ __device__ __forceinline__ void apply_op(cplx<R>* v, const FOp& op, const double
 // qubits FP64, 400 gates, k_fused 254 us without, 240 so).  The ops of a pass
 // lie one after the other, and behind the last one the program's buffer goes
 // on.
-template <class R>
+template <int AHEAD, class R>
 __device__ __forceinline__ void run_phase(cplx<R>* v, uint32_t begin, uint32_t end, const FOp* __restrict__ ops,
                                           const double* __restrict__ coef, uint32_t tb, uint64_t tile, FOp& next) {
     // the product of the phase's G factors (uniform, accumulated in FP64)
@@ -356,7 +356,7 @@ __device__ __forceinline__ void run_phase(cplx<R>* v, uint32_t begin, uint32_t e
             // set) the ratio table, both uniform loads; else each lane loads
             // its own variant
             if ((ea || eb) && op.dmode != 1) {
-                apply_d_lane<true>(v, c + 2 * kRegs * k, on);
+                apply_d_lane<AHEAD, true>(v, c + 2 * kRegs * k, on);
             } else {
                 const uint32_t var = ea ? 1u : 2u;
                 if (all) apply_d<false>(v, c, true);
@@ -604,7 +604,7 @@ __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPas
             exchange<kRegBits>(v, lds, cur, to);
             cur = to;
         }
-        run_phase(v, ph.op_begin, ph.op_end, ops, coef, tb, tile, next);
+        run_phase<(GATED || sizeof(R) == 8) ? 8 : 16>(v, ph.op_begin, ph.op_end, ops, coef, tb, tile, next);
     }
     Edge<R> out;
     out.set(pass, 1, !pass.permuted, tid);
@@ -635,8 +635,8 @@ __device__ __forceinline__ void fused_tile(cplx<R>* __restrict__ psi, const FPas
 
 // Four waves per SIMD: the exchange takes half a tile of LDS (32 KiB for
 // 2^12 FP64 or 2^13 FP32 amplitudes), and the op code keeps one copy of the
-// 16 amplitudes.  The persistent kernel's loop state does not fit beside
-// them in 128 registers: three.
+// 16 amplitudes.  The persistent kernel's loop state does not fit beside them
+// in 128 registers in FP64: three (137 VGPRs; FP32 takes 92, for five).
 #define QVNT_FUSED_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 #define QVNT_PERSIST_BOUNDS __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 3)))
 
@@ -710,9 +710,10 @@ __device__ __forceinline__ void persist_unit(cplx<R>* __restrict__ arena, const 
 
 // Units of each round (in thousandths) that blocks claim instead of taking
 // them in a fixed order, kPersistChunk consecutive units per claim
-// (4096-register batch, FP64: 54.2 ms per run with none; one unit per
-// claim: 51.6 with 100, 50.7 with 150, 53.1 with 250; with 150, two units
-// per claim 48.3, four 48.3; 300 in fours 48.3, 400 in fours 48.5).
+// (4096-register batch, FP64, when a tile took twice the LDS and two waves a
+// SIMD ran: 54.2 ms per run with none; one unit per claim: 51.6 with 100, 50.7
+// with 150, 53.1 with 250; with 150, two units per claim 48.3, four 48.3; 300
+// in fours 48.3, 400 in fours 48.5).
 constexpr uint32_t kPersistClaimed = 150;
 constexpr uint32_t kPersistChunk = 4;
 
@@ -733,13 +734,12 @@ constexpr uint32_t kPersistChunk = 4;
 // the end, after every block has left it; so the counters are zero again
 // when the launch ends.
 //
-// The dynamic LDS array starts 16-byte aligned after the claim word: the
-// tile's 16-byte accesses need it (an array at byte 4 made every run 35 %
-// slower).
+// The dynamic LDS array starts 16-byte aligned after the claim word (its
+// elements are 4 or 8 bytes; at byte 4 the FP64 ones would be misaligned).
 //
-// The launch bounds ask for no minimum of waves: the register allocation
-// stays at what the kernel uses, which is what the runtime's occupancy query (and so
-// the cooperative grid size) counts.
+// The launch bounds ask for one wave a SIMD at least and three at most, so
+// nothing pads the register allocation beyond what the kernel uses, which is
+// what the runtime's occupancy query (and so the cooperative grid size) counts.
 //
 // A launch that is not cooperative (a graph node whose cooperative
 // attribute the runtime did not honour) has no grid barrier: every block
