@@ -390,9 +390,10 @@ def tfim_pair_leg(n, steps, forms=("fused", "plain")):
 def serve_leg(requests, n_hi, slots, arena_gib, dense, plain=True, loads=(0.5, 0.8, 1.0), plain_requests=128):
     """Serving workload (n log-uniform in [12, n_hi], 100-2000 mixed gates,
     1024 seeded shots of measure_mask on 8 random qubits per request):
-      serial_plain   closed loop, one request at a time, plain form, on the
-                     first plain_requests requests (the plain form takes
-                     ~0.3 s a request);
+      serial_plain   closed loop, one request at a time, the server's plain
+                     form (one kernel per SingleOp, without the shared
+                     passes of QReg.apply), on the first plain_requests
+                     requests (~0.3 s a request);
       serial_fused   closed loop, one request at a time, fused form (its
                      circuits/s is the capacity c of serial service);
       saturation     every request submitted at once into the
@@ -871,8 +872,8 @@ def main():
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": load_traffic(kernel_name),
                 "traffic_source": "profiles/pmc_traffic.json (not measured in this run): rocprofv3 --pmc FETCH_SIZE "
                                   "x 2.000 (calibrated on k_leaf, which reads the 16 GiB state once and reports 8 GiB) "
-                                  "+ WRITE_SIZE x 1.000 (k_init), rz on qubit 12 of a 30-qubit FP64 register "
-                                  "(bench.py --workload plain-classes)",
+                                  "+ WRITE_SIZE x 1.000 (k_init), on a 30-qubit FP64 register: runs of one brickwork "
+                                  "layer, single gates on qubit 12 or 3 (the file names each case)",
                 "kernel": kernel_name, "launches": d["launches"], "avg_ms": round(avg_ms, 4),
                 "bytes_per_launch": per_launch_bytes,
                 "timing": "HIP events on the register's stream around every launch of the timed layers"}

@@ -280,7 +280,8 @@ typedef struct qvnt_request {
     uint32_t prec;            /* qvnt_prec                                     */
     uint64_t init_state;
     const qvnt_op* op;        /* copied at submit                              */
-    uint32_t fused;           /* 1: fused form (qvnt_reg_apply_fused); 0: plain */
+    uint32_t fused;           /* 1: fused form (qvnt_reg_apply_fused); 0: plain, one kernel per
+                                 SingleOp: qvnt_reg_apply's results without its shared passes */
     uint32_t max_qubits;      /* fused tile qubits, 0 = default                */
     uint32_t dense_min;       /* fused: dense-phase threshold, 0 = none (qvnt_reg_set_dense) */
     uint32_t reserved;        /* 0                                             */
@@ -321,8 +322,10 @@ enum qvnt_kclass {
     QVNT_K_DIAG = 0,   /* phase-only diagonal, single pass                */
     QVNT_K_PAIR,       /* 2-amplitude orbit (pair mix / permutation)      */
     QVNT_K_QUAD,       /* 4-amplitude orbit (H2, U2)                      */
-    QVNT_K_FUSED,      /* fused multi-gate tile pass                      */
-    QVNT_K_REDUCE,     /* |psi|^2 tree reduction                          */
+    QVNT_K_FUSED,      /* fused multi-gate tile pass, plain-form run      */
+    QVNT_K_REDUCE,     /* |psi|^2 tree reduction: one a norm; one for a
+                          call's draws from 2^12 amplitudes on (below,
+                          the draws make the sums themselves: OTHER)      */
     QVNT_K_COLLAPSE,   /* measurement collapse / rescale                  */
     QVNT_K_OTHER,
     QVNT_KCLASS_COUNT

@@ -34,7 +34,7 @@ COMMON = ["-std=c++17", "-O3", "-fPIC", "-Wall", "-Wno-unused-result",
 # memory; without the sinking every case keeps constant indices.  Their
 # branches are uniform over a wave, and left as they are (not structurized)
 # they keep one copy of the 16 amplitudes instead of an old and a new one: in
-# FP64 110 VGPRs instead of 218 (runs.hip), 113 instead of 221 (fused.hip).
+# FP64 120 VGPRs (k_run) and 114 (k_fused) instead of some 220.
 UNIFORM = ["-mllvm", "-simplifycfg-sink-common=false", "-mllvm", "-structurizecfg-skip-uniform-regions=true"]
 EXTRA = {"fused.hip": UNIFORM, "runs.hip": UNIFORM}
 

@@ -40,11 +40,13 @@ namespace fusion {
 
 constexpr int kRegBits = 4;                // register qubits per phase
 constexpr int kRegs = 1 << kRegBits;       // amplitudes per thread
-constexpr int kMaxTile = 13;               // t: at most 2^13 amplitudes per tile (64 KiB of LDS in FP32)
-// the largest tile whose amplitudes fit the kernel's 64 KiB LDS tile
+constexpr int kMaxTile = 13;               // t: at most 2^13 amplitudes per tile
+// the largest tile: one component of its amplitudes, which is what an
+// exchange moves through LDS at a time, fits 32 KiB
 constexpr unsigned max_tile(bool fp64) { return fp64 ? 12u : 13u; }
 // the default tile cap: 2^12 amplitudes in both precisions (an FP32 tile of
-// 2^13 is one 512-thread block per CU and measured slower on large states)
+// 2^13 measured slower on large states when it took 64 KiB of LDS and a CU
+// held one; not measured again since it takes 32 KiB)
 constexpr unsigned kDefaultTile = 12;
 constexpr int kMinFused = 6;               // below 2^6 amplitudes the plain kernels run
 constexpr int kMinDenseTile = 10;          // dense phases need whole 64-lane waves: 2^(t-4) >= 64
@@ -111,7 +113,8 @@ struct FOp {                // 64 bytes
 struct FPhase {
     uint32_t op_begin, op_end;
     uint32_t rpos[kRegBits];  // local positions of the register bits, ascending
-    uint32_t sroff[kRegs];    // swizzled LDS offset of register i (the swizzle is XOR-linear)
+    uint32_t sroff[kRegs];    // swizzled LDS offset of register i (the swizzle is XOR-linear); not read by the
+                              // kernels, which make their offsets from rpos (tile.hpp)
     uint32_t dense;           // 1: the phase is one 16x16 unitary on its register bits (matrix cores)
     uint32_t ucoef;           // dense: offset (in doubles) of U, row-major complex
 };
@@ -123,10 +126,12 @@ struct FPass {
     uint32_t direct_first;    // 1: the first phase's registers are local bits t-4..t-1
     uint32_t direct_last;     // 1: same for the last phase (0 when permuted)
     uint32_t tpos[kMaxTile];  // global positions of the local bits, ascending
-    uint64_t hoff[kRegs];     // global offset of local bits t-4..t-1 = j
+    uint64_t hoff[kRegs];     // global offset of local bits t-4..t-1 = j; not read by the kernels (top_global)
     // permuted: the pass ends with a permutation of its qubits (a relabeled
     // swap put back): the thread that stores local index L = tid + j * 2^(t-4)
-    // reads it from LDS offset (XOR over tid's set bits k of pimg[k]) ^ pout[j]
+    // reads the element behind the offset (XOR over tid's set bits k of
+    // pimg[k]) ^ pout[j].  The offsets are swizzled by lds_swizzle, its own
+    // inverse; the kernels undo it and apply their own swizzle.
     uint32_t permuted;
     uint32_t pimg[kMaxTile - kRegBits];
     uint32_t pout[kRegs];
@@ -153,8 +158,9 @@ struct BItem {              // 32 bytes
     uint32_t tiles;         // tiles of the pass
 };
 
-// LDS swizzle: bits 4..7 of the local index are XORed into bits 0..3, so
-// 16 lanes that differ in bits 4..7 hit 16 different 16-byte bank groups.
+// The swizzle of the program's offsets (sroff, pimg, pout): bits 4..7 of the
+// local index XORed into bits 0..3.  (The kernels' exchange has its own,
+// tile.hpp.)
 inline uint32_t lds_swizzle(uint32_t e) { return e ^ ((e >> 4) & 15u); }
 
 // A work unit of the persistent batched kernel: tiles [tile0, tile_end) of
@@ -200,10 +206,11 @@ uint64_t program_cost(const Program& prog);
 // kAutoTiles that fits the buffer, keeping the steps with the lowest
 // estimated run time: passes x a_t + program_cost x b_t (a plain step
 // counted as a pass), with a_t, b_t per tile size and precision fitted to
-// measured fused applies on MI355X.  Larger tiles need fewer passes;
-// smaller tiles run each op faster (more, smaller blocks per CU hide the
-// barriers between phases).  Returns the tile size kept.  (13 only in
-// FP32: an FP64 tile stops at 12, max_tile.)
+// fused applies on MI355X when the tile was exchanged whole through LDS, two
+// waves a SIMD; they put ten 30-qubit brickwork layers at 118 ms, which now
+// take 90.  Larger tiles need fewer passes; smaller tiles run each op faster
+// (more, smaller blocks per CU hide the barriers between phases).  Returns
+// the tile size kept.  (13 only in FP32: an FP64 tile stops at 12, max_tile.)
 constexpr unsigned kAutoTiles[] = {10, 11, 12, 13};
 // From 2^28 amplitudes a pass takes milliseconds, more than compiling the
 // candidates costs; single-register applies choose the tile from there.

@@ -110,7 +110,9 @@ Memory memory_of(const void* p);
 // own copy to pageable memory does one after the other: 20 qubits FP64,
 // probabilities 8 MiB 510 us, state 16 MiB 950 us; so 310 and 540 (the bus
 // alone: 155 and 310), in pieces of 256 KiB 400 and 730, of 1 MiB 390 and 670.
-// 10 qubits: 51 and 28 us, so 26 and 13.
+// 10 qubits: 51 and 28 us, so 26 and 13.  (States of 32 to 512 KiB take the
+// runtime 3 to 4 us less once it has its copy queue, 10.5 and 14.4 us for 32
+// KiB; making the queue takes the process's first call 6 ms.)
 // kNoBlock: no pinned memory, nothing done.
 constexpr size_t kHostChunk = size_t(512) << 10;
 constexpr int kNoBlock = -1;

@@ -6,18 +6,20 @@
 // below (4-6 us each from one to the next).  A run reads and writes the
 // state once for all its SingleOps, which leaves FP64 arithmetic beside the
 // HBM stream: a rz, rx or ry is 6 operations an amplitude.  Measured, one
-// call each, before (a kernel per SingleOp) and with runs:
-//   30-qubit brickwork layer, FP64, 106 SingleOps   576 ms    36 ms
-//   27-qubit Ising step, FP32, 135 SingleOps         45 ms   7.6 ms
+// whole call each with reset and readout, before (a kernel per SingleOp) and
+// with runs:
+//   30-qubit brickwork layer, FP64, 106 SingleOps   579 ms    41 ms (runs alone 31)
+//   27-qubit Ising step, FP32, 135 SingleOps         45 ms   7.4 ms
 //   15-qubit circuit, FP32, 300 gates               1.4 ms  0.26 ms
-//   10-qubit QFT with register and readback         241 us    48 us
+//   10-qubit QFT with register and readback         238 us    41 us
 //
 // From 22 qubits 256 threads hold a tile of 2^12 FP64 amplitudes in
 // registers, 16 each (2^13 in FP32: 512 threads); LDS only carries them from
 // one phase's layout to the next, one component at a time (32 KiB), so four
 // blocks fit a CU and, at 120 registers, four waves a SIMD: one block's HBM
-// accesses overlap the others' arithmetic, which bounds it (80 % of the
-// vector issue slots at 30 qubits).  Below, 8 amplitudes a thread and
+// accesses overlap the others' arithmetic, which bounds it: 30 qubits, a third
+// of a brickwork layer, 4.85e9 vector instructions on 1024 SIMDs in 10.8 ms,
+// four cycles each, 73 % of the cycles at 2.4 GHz.  Below, 8 amplitudes a thread and
 // smaller tiles (runs.hpp): there the time is each op's latency -- its load
 // from LDS, the dispatch, 16 or 8 amplitudes' dependent FP64 -- some 0.3 us.
 // The program comes with the launch as kernel arguments: no upload, no

@@ -53,7 +53,7 @@ constexpr unsigned max_tile(unsigned ns, bool fp64) { return ns <= kTinyQubits ?
 constexpr unsigned row_bits(bool fp64) { return fp64 ? 3u : 4u; }
 
 // Codes: a family and, where it has them, the register bits it works on
-// (one bit: j; two bits j0 < j1: pair_index).
+// (one bit: j; two bits j0 < j1: pair_variant).
 enum Family : uint32_t {
     F_PH = 0,      // phase (re, im) on the amplitudes of `pc`
     F_I1, F_I2, F_I3,  // i, -1, -i on the amplitudes of `pc`

@@ -10,7 +10,8 @@
 // caller's thread).  A slot's worker admits the first queued request that
 // fits the arena -- smaller requests may pass a large one at the head of
 // the queue, up to kMaxBypass times -- and enqueues its whole life on the
-// slot's stream: init, apply (fused or plain), measurement tree and draws,
+// slot's stream: init, apply (fused, or plain as one kernel per SingleOp,
+// without the runs of a register's plain apply), measurement tree and draws,
 // outcome copy, event.  It then waits for the event, returns the arena
 // block and posts the result.  Requests of 2^27 amplitudes or more run one
 // at a time (kBigQubits); smaller ones overlap with them and each other.  Workers enqueue in parallel, so a long
