@@ -74,3 +74,28 @@ def test_fused_permutations_equal_single_kernels(n, tq, prec):
         r.apply_fused(circ, max_qubits=tq)
         got = r.get_state()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n", [26, 27])
+def test_a_run_ends_before_gates_with_many_controls(n):
+    """FP32: the planner leaves gates with many controls behind a run to their
+    own kernels, after it has looked at them as part of it (more phases, more
+    tile qubits); between two stretches of other gates they stay in.  The same
+    bits as one SingleOp a call."""
+    plain, many = None, None
+    for k in range(14):
+        o = op.ry(0.2 + k, 1 << (4 + k % 7)) * op.rzz(0.3 + k, (1 << (4 + k % 7)) | (1 << (n - 1 - k % 3)))
+        plain = o if plain is None else plain * o
+    for k in range(30):
+        o = (op.rx if k % 2 else op.ry)(0.4 + k, 1 << (12 + k % 4)).c(0b11111 << (17 + k % 2))
+        many = o if many is None else many * o
+    start = op.h((1 << n) - 1)
+    for queue in (plain * many, plain * many * plain, many * plain):
+        with QReg(n, prec="f32") as run, QReg(n, prec="f32") as one:
+            run.apply(start)
+            one.apply(start)
+            run.apply(queue)
+            for k in range(len(queue)):
+                one.apply(queue[k])
+            a, b = run.get_state(), one.get_state()
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
